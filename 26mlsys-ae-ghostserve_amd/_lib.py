@@ -61,6 +61,24 @@ class ChunkStripe(C.Structure):
 
 _csp = C.POINTER(ChunkStripe)
 
+
+class KvBhtd(C.Structure):
+    """struct kvec_kv_bhtd of include/kvec.h."""
+    _fields_ = [
+        ("k", C.c_void_p),
+        ("v", C.c_void_p),
+        ("B", C.c_int64),
+        ("H", C.c_int64),
+        ("T", C.c_int64),
+        ("head_bytes", C.c_int64),
+        ("stride_b", C.c_int64),
+        ("stride_h", C.c_int64),
+        ("stride_t", C.c_int64),
+    ]
+
+
+_kbp = C.POINTER(KvBhtd)
+
 # name -> (restype, argtypes); mirrors include/kvec.h
 SIGNATURES = {
     "kvec_version": (_i, []),
@@ -89,6 +107,8 @@ SIGNATURES = {
     "kvec_unpack_kv": (_i, [_vp, _vp, _i, _i, _vp]),
     "kvec_gs_rdp_backup": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "kvec_gs_rdp_recover": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp]),
+    "kvec_gs_rdp_backup_kv": (_i, [_kbp, _vp, _i, _i, _i, _vp]),
+    "kvec_gs_rdp_recover_kv": (_i, [_vp, _kbp, _i, _i, _i, _i, _i, _vp]),
     "kvec_gs_pack_row": (_i, [_vp, _vp, _vp, _i64, _i, _i64, _vp]),
     "kvec_gs_rdp_parity": (_i, [_vp, _i, _i, _i, _vp]),
     "kvec_hook_step": (_i, [_kvp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _pp]),
@@ -134,6 +154,32 @@ def call(name: str, *args) -> int:
         msg = lib().kvec_last_error().decode(errors="replace")
         raise KvecError(f"{name} failed ({lib().kvec_strerror(rc).decode()}): {msg}")
     return rc
+
+
+EUNSUPPORTED = -2
+
+
+def call_if_built(name: str, *args) -> bool:
+    """`call`, returning False instead of raising when the entry point does not
+    take the layout (KVEC_EUNSUPPORTED: nothing was enqueued)."""
+    rc = getattr(lib(), name)(*args)
+    if rc == EUNSUPPORTED:
+        return False
+    if rc != 0:
+        msg = lib().kvec_last_error().decode(errors="replace")
+        raise KvecError(f"{name} failed ({lib().kvec_strerror(rc).decode()}): {msg}")
+    return True
+
+
+def kv_bhtd(k, v):
+    """The kvec_kv_bhtd of K and V tensors indexed [B, H, T, D], or None when
+    they differ in strides or a head's values are not adjacent."""
+    B, H, T, D = k.shape
+    ks, vs = k.stride(), v.stride()
+    if ks != vs or ks[3] != 1:
+        return None
+    es = k.element_size()
+    return KvBhtd(k.data_ptr(), v.data_ptr(), B, H, T, D * es, ks[0] * es, ks[1] * es, ks[2] * es)
 
 
 def ptr_array(tensors) -> C.Array:

@@ -1,0 +1,280 @@
+// gs_kv.hip -- the star-diagonal code's backup and recovery straight from and
+// to K and V tensors indexed [B][H][T][D].
+//
+// The reference's wrappers permute K and V to token-major copies, pack those
+// into the rows and code the rows (benchmark/rdp/main.py:44-92); recovery
+// copies the rows out and permutes back (:95-126).  Here the coding kernels
+// address the token-major stream in K and V (kv_stream.h), so each byte of K
+// and V crosses HBM once.  Bound by HBM: 16 requests x 8 heads x 2047 tokens x
+// 128 (bf16, six data rows), kernel trace: backup 56 us (5.6 TB/s of the 313
+// MB it must move), recovery 58 us (5.0 TB/s of 291 MB; a wave's 1 KiB of
+// stream is four heads, so its stores to K and V are four 256-byte pieces),
+// where the torch permutes alone took 99 us beside a 53 us coding kernel.
+// Whole calls, A/B: recovery 169 -> 84 us, the reference demo's backup (1 x 8
+// x 512 x 128, eight rows) 48 -> 32 us.
+#include "gs_star.h"
+#include "kv_stream.h"
+
+namespace kvec {
+
+// ------------------------------------------------------------------- backup
+// One tile of 16 BS bytes of every row: the ND data rows are the stream
+// K || V || zeros laid end to end, row r at stream byte r Sb, and each lane
+// loads the aligned stream chunk under its window of every row, all requested
+// at once.  It stores the chunk into the data rows (the rows start 16-byte
+// aligned, so a stream chunk is a row chunk) and takes the P window (mr bytes
+// into the chunk) and the Q window (2 r bytes before that) from it and a
+// neighbour lane's chunk by DPP shifts; with ND <= 8 the Q window starts at
+// most 14 bytes before the chunk.  Lane 63 loads the chunk after the wave's
+// and lane 0 the one before it into one register set, the edge value of both
+// shifts.  P and Q go through LDS to tile_store.
+// Q words 0 .. ND-2 wrap: block 0's first threads compute each from its ND
+// words, requested before the rows, and they replace what the shifts gave.
+template <int ND, int BS, bool FLAT>
+__global__ __launch_bounds__(BS) void gs_backup_kv_kernel(KvStream src, uint8_t* sh, uint32_t Sb, GsStar star) {
+    constexpr uint32_t TB = 16 * BS;
+    __shared__ __attribute__((aligned(16))) uint8_t tp[TB + 16];
+    __shared__ __attribute__((aligned(16))) uint8_t tq[TB + 16];
+    const uint32_t t0 = blockIdx.x * TB;
+    const uint32_t nbytes = Sb - t0 < TB ? Sb - t0 : TB;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t w64 = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))) * 1024;
+    const uint32_t data_end = uint32_t(ND) * Sb;
+    const KvReader<FLAT> in(src);
+    auto row_m = [&](int r) { return (uint32_t(r) * Sb + t0) & 15; };
+    auto row_x0 = [&](int r) { return uint32_t(r) * Sb + t0 - row_m(r); };
+    // wrapped Q words
+    const bool wraps = ND > 1 && t0 == 0 && threadIdx.x < ND - 1;
+    uint16_t wq[ND];
+    if (wraps) {
+        const uint32_t d = threadIdx.x, S = Sb / 2;
+#pragma unroll
+        for (int r = 0; r < ND; ++r) wq[r] = in.word(2 * (uint32_t(r) * S + (d >= uint32_t(r) ? d - r : S + d - r)));
+    }
+    // lanes whose chunk holds no byte any window of the row uses load nothing
+    const bool live = 16 * threadIdx.x < nbytes + 16;
+    u32x4 c0[ND], e[ND];
+#pragma unroll
+    for (int r = 0; r < ND; ++r) {
+        const uint32_t mr = row_m(r), x0 = row_x0(r), X = x0 + 16 * threadIdx.x;
+        const int s = int(mr) - 2 * r;
+        const uint32_t lo = x0 + w64;   // the wave's chunks, and one on each side
+        const auto f = in.from(lo >= 16 ? lo - 16 : 0, lo + 1024 + 16);
+        c0[r] = in.load(X, live, f);
+        const bool want = (lane == 63 && (mr > 0 || s > 0)) || (lane == 0 && s < 0 && X != 0);
+        e[r] = in.load(lane == 63 ? X + 16 : X - 16, live && want, f);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int32_t w0 = int32_t((t0 >> 1) + 8 * threadIdx.x);
+    u32x4 p = {0, 0, 0, 0}, q = {0, 0, 0, 0};
+#pragma unroll
+    for (int r = 0; r < ND; ++r) {
+        const uint32_t mr = row_m(r), x0 = row_x0(r), X = x0 + 16 * threadIdx.x;
+        const int s = int(mr) - 2 * r;
+        const u32x4 c1 = from_next_lane_or(c0[r], e[r]), cm = from_prev_lane_or(c0[r], e[r]);
+        // The chunk into the data rows: non-temporal, except in the two
+        // 128-byte lines the wave shares with its neighbours (copy_chunk_split).
+        // In the row's last tile the last thread also stores the chunk after its
+        // own, which a row ending with the tile can end in.
+        const uint32_t rend = uint32_t(r + 1) * Sb;
+        const uint32_t pre = ((uint32_t(reinterpret_cast<uintptr_t>(sh)) + x0) >> 4) & 7;
+        const bool edge = pre != 0 && (lane < 8 - pre || lane >= 64 - pre);
+        auto put = [&](uint32_t at, u32x4 v, bool shared) {
+            if (at + 16 <= data_end) {
+                if (shared) st16(sh + at, v);
+                else st_stream(sh, at, v);
+            } else if (at < data_end) {
+                const gptr<uint8_t> d = as_global(sh);
+                for (uint32_t i = 0; i < data_end - at; ++i) d[at + i] = byte_of(v, int(i));
+            }
+        };
+        if (X < rend) put(X, c0[r], edge);
+        if (t0 + TB >= Sb && mr > 0 && threadIdx.x == BS - 1 && X + 16 < rend) put(X + 16, c1, true);
+        p ^= mr ? funnel16(c0[r], c1, mr) : c0[r];
+        u32x4 qw;
+        if (s > 0) qw = funnel16(c0[r], c1, uint32_t(s));
+        else if (s == 0) qw = c0[r];
+        else qw = funnel16(cm, c0[r], uint32_t(s + 16));
+        q ^= star.d[r] < 0 ? qw : drop_word(qw, int64_t(star.d[r]) - w0);
+    }
+    *reinterpret_cast<u32x4*>(tp + 16 * threadIdx.x) = p;
+    *reinterpret_cast<u32x4*>(tq + 16 * threadIdx.x) = q;
+    __syncthreads();
+    if (ND > 1 && t0 == 0) {
+        if (wraps) {
+            uint16_t v = 0;
+#pragma unroll
+            for (int r = 0; r < ND; ++r) v ^= star.d[r] == int32_t(threadIdx.x) ? uint16_t(0) : wq[r];
+            *reinterpret_cast<uint16_t*>(tq + 2 * threadIdx.x) = v;
+        }
+        __syncthreads();
+    }
+    tile_store<true, BS>(sh + data_end + t0, tp, nbytes);
+    tile_store<true, BS>(sh + data_end + Sb + t0, tq, nbytes);
+}
+
+// ----------------------------------------------------------------- recovery
+// Row t (t >= 0) rebuilt as P ^ the other data rows, written back into the
+// shards, and the stream written to K and V.  A block owns one tile of every
+// row.  A surviving row's aligned chunks lie in one piece of K or V, so they
+// go there straight from the registers they were loaded into; its at most 15
+// bytes before the first and after the last whole chunk go byte by byte from
+// block 0.  The rebuilt row is formed at the row's own alignment and goes
+// through LDS.  Row t itself is never read.
+template <int ND, int BS, bool FLAT>
+__global__ __launch_bounds__(BS) void gs_recover_kv_kernel(uint8_t* sh, uint32_t Sb, uint32_t in_bytes, int t,
+                                                           KvStream dst) {
+    constexpr uint32_t TB = 16 * BS;
+    __shared__ __attribute__((aligned(16))) uint8_t tile[TB + 16];
+    const uint32_t t0 = blockIdx.x * TB;
+    const uint32_t nbytes = Sb - t0 < TB ? Sb - t0 : TB;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t out_len = 2 * dst.kb;
+    const __amdgpu_buffer_rsrc_t rs = chunk_rsrc(sh, (in_bytes + 15) & ~15u);
+    // batch row i: data row i, or i + 1 from row t on (then P last)
+    auto row_of = [&](int i) { return i + (t >= 0 && i >= t ? 1 : 0); };
+    auto row_a = [&](int i) { return uint32_t(row_of(i)) * Sb + t0; };
+    const bool live = 16 * threadIdx.x < nbytes + 16;
+    u32x4 lo[ND], e1[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const uint32_t A = row_a(i), m = A & 15, my = A - m + 16 * threadIdx.x;
+        lo[i] = chunk_load(rs, live ? my : kNoLoad);
+        e1[i] = chunk_load(rs, live && lane == 63 && m ? my + 16 : kNoLoad);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto put_byte = [&](uint32_t x, uint8_t b) {
+        if (x < out_len) *as_global(kv_at<FLAT>(dst, x)) = b;
+    };
+    u32x4 acc = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const uint32_t A = row_a(i), m = A & 15, X = A - m + 16 * threadIdx.x;
+        acc ^= m ? funnel16(lo[i], from_next_lane_or(lo[i], e1[i]), m) : lo[i];
+        const uint32_t r0 = A - t0;
+        if (row_of(i) < ND && X >= r0 && X + 16 <= r0 + Sb && X + 16 <= out_len)
+            st_stream(kv_at<FLAT>(dst, X), 0, lo[i]);
+    }
+    if (blockIdx.x == 0) {
+        for (uint32_t u = threadIdx.x; u < 32 * ND; u += BS) {
+            const uint32_t j = uint32_t(row_of(int(u >> 5))), b = u & 31;
+            const uint32_t r0 = j * Sb, r1 = r0 + Sb, first = (r0 + 15) & ~15u;
+            const uint32_t x = b < 16 ? r0 + b : (r1 & ~15u) + (b - 16);
+            const bool mine = b < 16 ? x < first && x < r1 : x >= first && x < r1;
+            if (j < uint32_t(ND) && mine) put_byte(x, as_global(sh)[x]);
+        }
+    }
+    if (t < 0) return;
+    *reinterpret_cast<u32x4*>(tile + 16 * threadIdx.x) = acc;
+    __syncthreads();
+    tile_store<false, BS>(sh + uint32_t(t) * Sb + t0, tile, nbytes);
+    // the same bytes to K and V
+    const uint32_t D0 = uint32_t(t) * Sb + t0, E = D0 + nbytes;
+    const uint32_t A0 = (D0 + 15) & ~15u, A1 = E & ~15u;
+    if (A0 < A1) {
+        const uint32_t sh0 = A0 - D0;   // < 16
+        for (uint32_t k = threadIdx.x; k < (A1 - A0) >> 4; k += BS) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(tile + 16 * k);
+            if (sh0) v = funnel16(v, *reinterpret_cast<const u32x4*>(tile + 16 * k + 16), sh0);
+            const uint32_t X = A0 + 16 * k;
+            if (X + 16 <= out_len) st_stream(kv_at<FLAT>(dst, X), 0, v);
+        }
+        const uint32_t i = threadIdx.x;
+        if (i < 16 && D0 + i < A0) put_byte(D0 + i, tile[i]);
+        else if (i >= 16 && i < 32 && A1 + (i - 16) < E) put_byte(A1 + (i - 16), tile[A1 + (i - 16) - D0]);
+    } else {
+        for (uint32_t x = D0 + threadIdx.x; x < E; x += BS) put_byte(x, tile[x - D0]);
+    }
+}
+
+// ---------------------------------------------------------------- host side
+// Threads per tile: 512 (8 KiB tiles), or 128 where those would leave most of
+// the 256 compute units idle.
+constexpr int kKvBS = 512, kKvSmallBS = 128;
+constexpr uint64_t kKvSmallTiles = 512;
+
+typedef void (*BackupKvFn)(KvStream, uint8_t*, uint32_t, GsStar);
+typedef void (*RecoverKvFn)(uint8_t*, uint32_t, uint32_t, int, KvStream);
+
+template <int BS, bool FLAT, int ND = 1>
+static BackupKvFn backup_kv_fn(int nd) {
+    if constexpr (ND > 8) {
+        return nullptr;
+    } else {
+        if (nd == ND) return &gs_backup_kv_kernel<ND, BS, FLAT>;
+        return backup_kv_fn<BS, FLAT, ND + 1>(nd);
+    }
+}
+template <int BS, bool FLAT, int ND = 1>
+static RecoverKvFn recover_kv_fn(int nd) {
+    if constexpr (ND > 8) {
+        return nullptr;
+    } else {
+        if (nd == ND) return &gs_recover_kv_kernel<ND, BS, FLAT>;
+        return recover_kv_fn<BS, FLAT, ND + 1>(nd);
+    }
+}
+
+static bool small_tiles(uint64_t Sb) { return (Sb + 16 * kKvBS - 1) / (16 * kKvBS) < kKvSmallTiles; }
+
+// Whether the K/V kernels take this stripe: 1..8 data rows of at least 64
+// words holding all of K and V, in a 16-byte-aligned tensor below 2 GiB.
+static bool kv_rows_ok(const KvStream& s, const void* shards, int nd, int64_t S) {
+    if (nd < 1 || nd > 8 || S < 64 || !aligned16(shards)) return false;
+    const uint64_t Sb = uint64_t(S) * 2;
+    return uint64_t(nd + 2) * Sb <= (uint64_t(1) << 31) - 16 && 2 * uint64_t(s.kb) <= uint64_t(nd) * Sb;
+}
+
+static KvDims gs_dims(const kvec_kv_bhtd* kv) {
+    return KvDims{kv->B, kv->H, kv->T, kv->head_bytes, kv->stride_b, kv->stride_h, kv->stride_t};
+}
+
+}  // namespace kvec
+
+using namespace kvec;
+
+extern "C" int kvec_gs_rdp_backup_kv(const kvec_kv_bhtd* kv, void* shards, int nd, int S, int star_base,
+                                     void* stream) {
+    static const char* fn = "kvec_gs_rdp_backup_kv";
+    if (!kv || !shards) return set_error(KVEC_EINVAL, "%s: null pointer", fn);
+    KvStream s{};
+    bool flat = false;
+    if (!make_kv_stream(&s, &flat, kv->k, kv->v, gs_dims(kv)) || !kv_rows_ok(s, shards, nd, S))
+        return set_error(KVEC_EUNSUPPORTED, "%s: layout or stripe not built", fn);
+    if (!kv->k || !kv->v) return set_error(KVEC_EINVAL, "%s: null K or V", fn);
+    const uint64_t Sb = uint64_t(S) * 2;
+    const Span w = {shards, uint64_t(nd + 2) * Sb, "shards", -1};
+    const Span r[2] = {{kv->k, s.ext, "k", -1}, {kv->v, s.ext, "v", -1}};
+    if (int rc = check_no_alias(&w, 1, r, 2, fn)) return rc;
+    const GsStar star = make_gs_star(star_base, S);
+    const bool small = small_tiles(Sb);
+    const BackupKvFn f = small ? (flat ? backup_kv_fn<kKvSmallBS, true>(nd) : backup_kv_fn<kKvSmallBS, false>(nd))
+                               : (flat ? backup_kv_fn<kKvBS, true>(nd) : backup_kv_fn<kKvBS, false>(nd));
+    const int bs = small ? kKvSmallBS : kKvBS;
+    hipLaunchKernelGGL(f, dim3(blocks_for(int64_t(Sb), 16 * bs)), dim3(bs), 0, as_stream(stream), s, (uint8_t*)shards,
+                       uint32_t(Sb), star);
+    return check_launch(fn);
+}
+
+extern "C" int kvec_gs_rdp_recover_kv(void* shards, const kvec_kv_bhtd* kv, int nd, int S, int star_base, int missing_a,
+                                      int missing_b, void* stream) {
+    static const char* fn = "kvec_gs_rdp_recover_kv";
+    if (!kv || !shards) return set_error(KVEC_EINVAL, "%s: null pointer", fn);
+    KvStream s{};
+    bool flat = false;
+    if (!make_kv_stream(&s, &flat, kv->k, kv->v, gs_dims(kv)) || !kv_rows_ok(s, shards, nd, S))
+        return set_error(KVEC_EUNSUPPORTED, "%s: layout or stripe not built", fn);
+    if (!kv->k || !kv->v) return set_error(KVEC_EINVAL, "%s: null K or V", fn);
+    const uint64_t Sb = uint64_t(S) * 2;
+    int t = -1;
+    if (int rc = gs_recover_row(nd, S, star_base, missing_a, missing_b, fn, &t)) return rc;
+    const Span w[3] = {{shards, uint64_t(nd + 2) * Sb, "shards", -1}, {kv->k, s.ext, "k", -1}, {kv->v, s.ext, "v", -1}};
+    if (int rc = check_no_alias(w, 3, nullptr, 0, fn)) return rc;
+    const bool small = small_tiles(Sb);
+    const RecoverKvFn f = small ? (flat ? recover_kv_fn<kKvSmallBS, true>(nd) : recover_kv_fn<kKvSmallBS, false>(nd))
+                                : (flat ? recover_kv_fn<kKvBS, true>(nd) : recover_kv_fn<kKvBS, false>(nd));
+    const int bs = small ? kKvSmallBS : kKvBS;
+    hipLaunchKernelGGL(f, dim3(blocks_for(int64_t(Sb), 16 * bs)), dim3(bs), 0, as_stream(stream), (uint8_t*)shards,
+                       uint32_t(Sb), uint32_t(uint64_t(nd + 1) * Sb), t, s);
+    return check_launch(fn);
+}

@@ -7,6 +7,7 @@
 // The column work runs on the tile engine (tile_engine.h).  The diagonal
 // parity Q[d] = XOR_r D_r[(d - r) mod S] skips each row's star word in the
 // same pass: the lane whose window holds it masks it before the XOR.
+#include "gs_star.h"
 #include "tile_engine.h"
 
 namespace kvec {
@@ -246,32 +247,6 @@ __global__ __launch_bounds__(kKvTB) void xor_encode_kv_kernel(const uint8_t* K, 
 // (C remainder: negative means no skip) out of the diagonal it lies on,
 // d = star_r + r (mod S).  That word is the one at position d - w0 of the
 // thread's row-r diagonal window, so it is masked there.
-// x % S with C semantics (the sign of x), dividing only when x is outside [0, S).
-__device__ __forceinline__ int64_t cmod(int64_t x, int64_t S) {
-    return (x >= 0 && x < S) ? x : x % S;
-}
-
-// v with its bytes 0..n-1 zeroed (n <= 0: v).
-__device__ __forceinline__ u32x4 drop_low_bytes(u32x4 v, int n) {
-    auto m = [&](int d) {
-        const int k = n - 4 * d;   // bytes of dword d to clear
-        return k <= 0 ? 0xFFFFFFFFu : (k >= 4 ? 0u : 0xFFFFFFFFu << (8 * k));
-    };
-    return u32x4{v.x & m(0), v.y & m(1), v.z & m(2), v.w & m(3)};
-}
-
-__device__ __forceinline__ u32x4 drop_word(u32x4 v, int64_t k) {
-    if (k < 0 || k >= 8) return v;
-    const uint32_t m = (k & 1) ? 0x0000FFFFu : 0xFFFF0000u;
-    switch (k >> 1) {
-        case 0: v.x &= m; break;
-        case 1: v.y &= m; break;
-        case 2: v.z &= m; break;
-        default: v.w &= m; break;
-    }
-    return v;
-}
-
 // Where the data rows' bytes come from.  Without K/V (FUSED false) they are
 // the shard rows themselves.  For the fused backup (the pack of
 // benchmark/rdp/kernel.cu:32-72, then the parity of :76-107) data-row bytes
@@ -362,15 +337,6 @@ __device__ __forceinline__ void gs_store_chunk32(uint8_t* base, uint32_t X, u32x
     for (int i = 0; i < 16; ++i)
         if (X + i < lim) d[X + i] = byte_of(v, i);
 }
-
-// Per data row r < 8: the diagonal its star word lies on, (star_r + r) mod S
-// with star_r = (star_base + r) % S, or -1 when the row skips nothing (C
-// remainder: a negative star_base gives a negative star_r).  The same for
-// every tile, so the host computes it once; the batched path runs only on
-// row tensors below 2 GiB, so it fits 32 bits.
-struct GsStar {
-    int32_t d[8];
-};
 
 // P/Q of one tile of a stripe of at least one full tile with ND = nd <= 8
 // data rows: each row's chunk, and the edge lanes' neighbour chunks, are all
@@ -832,11 +798,7 @@ static int gs_rdp_parity(uint16_t* sh, int nd, int64_t S, int star_base, hipStre
     const uint64_t lim = (uint64_t(1) << 31) - 16;
     const bool small = rows_bytes <= lim && (!fused || uint64_t(fused->kb) <= lim);
     const uint64_t rb = small ? rows_bytes : 0;
-    GsStar star{};
-    for (int r = 0; r < 8; ++r) {
-        const int64_t sr = (int64_t(star_base) + r) % S;
-        star.d[r] = sr < 0 ? -1 : int32_t((sr + r) % S);
-    }
+    const GsStar star = make_gs_star(star_base, S);
     if (fused)
         hipLaunchKernelGGL(gs_parity_fn<true>(nd), grid, dim3(kTB), 0, st, sh, nd, S, star_base, *fused, rb,
                            star);
@@ -844,6 +806,33 @@ static int gs_rdp_parity(uint16_t* sh, int nd, int64_t S, int star_base, hipStre
         hipLaunchKernelGGL(gs_parity_fn<false>(nd), grid, dim3(kTB), 0, st, sh, nd, S, star_base,
                            GsSource{nullptr, nullptr, 0, 0, 0}, rb, star);
     return check_launch(what);
+}
+
+// The data row a recovery rebuilds (*row, or -1) for the reported losses, as
+// the reference's launcher picks it (benchmark/rdp/kernel.cu:402-507): indices
+// outside [0, nd) are dropped, of two rows the lower one is rebuilt.
+int gs_recover_row(int nd, int S, int star_base, int missing_a, int missing_b, const char* fn, int* row) {
+    int a = (missing_a >= 0 && missing_a < nd) ? missing_a : -1;
+    int b = (missing_b >= 0 && missing_b < nd) ? missing_b : -1;
+    // Two rows lost: the reference's fill_a_star_from_P (benchmark/rdp/kernel.cu:268-282,
+    // launched at :466) reads P and the other rows at column (star_base + a) % S and writes
+    // row a there, a the lower row.  A negative remainder (C's %) addresses the row before
+    // each one, and before the tensor for row 0: undefined, so refused.  Otherwise that
+    // write lands in row a, which rebuild_row_from_P rewrites, and star_base changes no
+    // output byte.
+    if (a >= 0 && b >= 0 && a != b && S > 0 && (int64_t(star_base) + (a < b ? a : b)) % S < 0)
+        return set_error(KVEC_EINVAL,
+                         "%s: (star_base + a) %% S < 0 for lost rows %d and %d (star_base=%d): "
+                         "the reference addresses outside row a", fn, a < b ? a : b, a < b ? b : a, star_base);
+    int t = -1;
+    if (a >= 0 && b >= 0 && a != b)
+        t = a < b ? a : b;
+    else if (a >= 0 && b < 0)
+        t = a;
+    else if (b >= 0 && a < 0)
+        t = b;
+    *row = t;
+    return KVEC_OK;
 }
 
 }  // namespace kvec
@@ -1056,25 +1045,8 @@ extern "C" int kvec_gs_rdp_recover(void* shards, void* out_TN, int nd, int S, in
                                    int star_base, int missing_a, int missing_b, void* stream) {
     if (!shards) return set_error(KVEC_EINVAL, "kvec_gs_rdp_recover: null shards");
     hipStream_t st = as_stream(stream);
-    int a = (missing_a >= 0 && missing_a < nd) ? missing_a : -1;
-    int b = (missing_b >= 0 && missing_b < nd) ? missing_b : -1;
-    // Two rows lost: the reference's fill_a_star_from_P (benchmark/rdp/kernel.cu:268-282,
-    // launched at :466) reads P and the other rows at column (star_base + a) % S and writes
-    // row a there, a the lower row.  A negative remainder (C's %) addresses the row before
-    // each one, and before the tensor for row 0: undefined, so refused.  Otherwise that
-    // write lands in row a, which rebuild_row_from_P rewrites, and star_base changes no
-    // output byte.
-    if (a >= 0 && b >= 0 && a != b && S > 0 && (int64_t(star_base) + (a < b ? a : b)) % S < 0)
-        return set_error(KVEC_EINVAL,
-                         "kvec_gs_rdp_recover: (star_base + a) %% S < 0 for lost rows %d and %d (star_base=%d): "
-                         "the reference addresses outside row a", a < b ? a : b, a < b ? b : a, star_base);
     int t = -1;
-    if (a >= 0 && b >= 0 && a != b)
-        t = a < b ? a : b;
-    else if (a >= 0 && b < 0)
-        t = a;
-    else if (b >= 0 && a < 0)
-        t = b;
+    if (int rc = gs_recover_row(nd, S, star_base, missing_a, missing_b, "kvec_gs_rdp_recover", &t)) return rc;
     const bool copy_out = T > 0 && n > 0 && nd > 0 && S > 0;
     if (copy_out && !out_TN) return set_error(KVEC_EINVAL, "kvec_gs_rdp_recover: null output");
     const uint64_t total = 2 * uint64_t(T > 0 ? T : 0) * uint64_t(n > 0 ? n : 0);

@@ -111,8 +111,6 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
     B, H, T, D = keys_bhtd.shape
     n = B * H * D
     total_words = 2 * T * n
-    K_TN = keys_bhtd.permute(2, 0, 1, 3).contiguous().view(T, n)
-    V_TN = values_bhtd.permute(2, 0, 1, 3).contiguous().view(T, n)
 
     nd = int(num_data_shards)
     p = spec_prime(nd) if scheme == "spec" else 0
@@ -120,22 +118,31 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
         shard_size, pad_words = spec_shard_size_words(total_words, nd, p)
     else:
         shard_size, pad_words = determine_shard_size_words(total_words, nd)
-    shards = torch.empty((nd + 2, shard_size), dtype=torch.uint16, device=K_TN.device)
-    # the reference zero-fills everything; only the padding words are read
-    # before being written
-    shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
+    device = keys_bhtd.device
+    shards = torch.empty((nd + 2, shard_size), dtype=torch.uint16, device=device)
     t0 = torch.cuda.Event(enable_timing=True)
     t1 = torch.cuda.Event(enable_timing=True)
     t0.record()
-    if scheme == "spec":
-        # K_TN || V_TN into the data rows, then textbook RDP over the rows
-        _lib.call("kvec_rs16_pack", K_TN.data_ptr(), V_TN.data_ptr(), shards.data_ptr(),
-                  T * n, T * n, _stream(shards))
-        rows = _rows_u8(shards)
-        spec.rdp_encode(rows[:nd], rows[nd], rows[nd + 1], p, unit_bytes=spec.RDP_UNIT)
-    else:
-        rdp_kernel.fused_backup_full_kv(K_TN, V_TN, shards, nd, int(shard_size), int(T), int(n),
-                                        int(star_base))
+    # one pass over K and V where they lie, when their layout allows it; else
+    # token-major copies, then the pack and the code
+    kv = _lib.kv_bhtd(keys_bhtd, values_bhtd) if scheme == "ghostserve" else None
+    if kv is None or not _lib.call_if_built("kvec_gs_rdp_backup_kv", kv, shards.data_ptr(), nd,
+                                            int(shard_size), int(star_base), _stream(shards)):
+        K_TN = keys_bhtd.permute(2, 0, 1, 3).contiguous().view(T, n)
+        V_TN = values_bhtd.permute(2, 0, 1, 3).contiguous().view(T, n)
+        # the reference zero-fills everything; only the padding words are read
+        # before being written
+        shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
+        t0.record()
+        if scheme == "spec":
+            # K_TN || V_TN into the data rows, then textbook RDP over the rows
+            _lib.call("kvec_rs16_pack", K_TN.data_ptr(), V_TN.data_ptr(), shards.data_ptr(),
+                      T * n, T * n, _stream(shards))
+            rows = _rows_u8(shards)
+            spec.rdp_encode(rows[:nd], rows[nd], rows[nd + 1], p, unit_bytes=spec.RDP_UNIT)
+        else:
+            rdp_kernel.fused_backup_full_kv(K_TN, V_TN, shards, nd, int(shard_size), int(T),
+                                            int(n), int(star_base))
     t1.record()
     torch.cuda.synchronize()
     backup_ms = t0.elapsed_time(t1)
@@ -168,24 +175,36 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
     B, H, _, D = pkg["shape_BHTD"]
     dtype = pkg.get("dtype", torch.float16)
 
-    packed_TN = torch.empty(2 * T * n, dtype=dtype, device=shards.device)
+    kv_shape = (int(B), int(H), int(T), int(D))
+    keys = torch.empty(kv_shape, dtype=dtype, device=shards.device)
+    values = torch.empty(kv_shape, dtype=dtype, device=shards.device)
+    _lib.require_cuda(shards, keys, values, what="fused_recovery_full_kv tensor")
     t0 = torch.cuda.Event(enable_timing=True)
     t1 = torch.cuda.Event(enable_timing=True)
     t0.record()
-    if pkg.get("scheme", "ghostserve") == "spec":
-        lost = [int(e) for e in (missing_a, missing_b) if 0 <= int(e) < nd + 2]
-        spec.rdp_decode(_rows_u8(shards), int(pkg["p"]), lost, unit_bytes=spec.RDP_UNIT)
-        _lib.call("kvec_rs16_split", shards.data_ptr(), packed_TN.data_ptr(),
-                  packed_TN[T * n:].data_ptr(), T * n, T * n, _stream(shards))
-    else:
-        rdp_kernel.fused_recovery_full_kv(shards, packed_TN, int(nd), int(shard_size), int(T),
-                                          int(n), int(star_base), int(missing_a), int(missing_b))
+    # the rows written straight to K and V when the layout allows it; else
+    # through a token-major copy
+    direct = (pkg.get("scheme", "ghostserve") != "spec" and
+              _lib.call_if_built("kvec_gs_rdp_recover_kv", shards.data_ptr(),
+                                 _lib.kv_bhtd(keys, values), int(nd), int(shard_size),
+                                 int(star_base), int(missing_a), int(missing_b), _stream(shards)))
+    if not direct:
+        packed_TN = torch.empty(2 * T * n, dtype=dtype, device=shards.device)
+        if pkg.get("scheme", "ghostserve") == "spec":
+            lost = [int(e) for e in (missing_a, missing_b) if 0 <= int(e) < nd + 2]
+            spec.rdp_decode(_rows_u8(shards), int(pkg["p"]), lost, unit_bytes=spec.RDP_UNIT)
+            _lib.call("kvec_rs16_split", shards.data_ptr(), packed_TN.data_ptr(),
+                      packed_TN[T * n:].data_ptr(), T * n, T * n, _stream(shards))
+        else:
+            rdp_kernel.fused_recovery_full_kv(shards, packed_TN, int(nd), int(shard_size), int(T),
+                                              int(n), int(star_base), int(missing_a),
+                                              int(missing_b))
     t1.record()
+    if not direct:
+        dK = packed_TN[:T * n].view(T, n)
+        dV = packed_TN[T * n:].view(T, n)
+        keys.copy_(dK.view(T, B, H, D).permute(1, 2, 0, 3))
+        values.copy_(dV.view(T, B, H, D).permute(1, 2, 0, 3))
     torch.cuda.synchronize()
     recover_ms = t0.elapsed_time(t1)
-
-    dK = packed_TN[:T * n].view(T, n)
-    dV = packed_TN[T * n:].view(T, n)
-    keys = dK.view(T, B, H, D).permute(1, 2, 0, 3).contiguous()
-    values = dV.view(T, B, H, D).permute(1, 2, 0, 3).contiguous()
     return keys, values, {"recover_ms": recover_ms}

@@ -40,8 +40,9 @@ extern "C" {
  * kvec_version() / 10000 == KVEC_VERSION / 10000 before its first call.
  * 1.0.0: kvec_rdp_encode / kvec_rdp_decode / kvec_rdp_encode_paged take
  * unit_bytes, kvec_chunk_stripe has region_off and unit_bytes (0.1.0 had
- * neither).  1.1.0: kvec_hook_step added. */
-#define KVEC_VERSION 10100
+ * neither).  1.1.0: kvec_hook_step added.  1.2.0: the *_kv entry points over
+ * kvec_kv_bhtd added. */
+#define KVEC_VERSION 10200
 int kvec_version(void);
 /* Static description of a KVEC_E* code. */
 const char* kvec_strerror(int code);
@@ -252,6 +253,27 @@ int kvec_gs_rdp_backup(const void* K_TN, const void* V_TN, void* shards, int nd,
  * writes outside row a (:268-282); that case returns KVEC_EINVAL. */
 int kvec_gs_rdp_recover(void* shards, void* out_TN, int nd, int S, int T, int n, int star_base,
                         int missing_a, int missing_b, void* stream);
+/* K and V tensors of 16-bit words indexed [B][H][T][head], each head's
+ * head_bytes contiguous; the two share their strides (bytes). */
+typedef struct kvec_kv_bhtd {
+    void* k;
+    void* v;
+    int64_t B, H, T;
+    int64_t head_bytes;
+    int64_t stride_b, stride_h, stride_t;
+} kvec_kv_bhtd;
+
+/* fused_backup_full_kv, benchmark/rdp/main.py:44-92, without its permuted
+ * copies: the data rows are the token-major stream K [T][B][H][head] || V ||
+ * zeros read from K and V where they lie, then P and Q as kvec_gs_rdp_backup.
+ * Every byte of shards is written.  KVEC_EUNSUPPORTED, with nothing enqueued,
+ * for layouts it does not take: head_bytes, strides or pointers not multiples
+ * of 16, nd > 8, S < 64, K or V over 1 GiB, shards of 2 GiB. */
+int kvec_gs_rdp_backup_kv(const kvec_kv_bhtd* kv, void* shards, int nd, int S, int star_base, void* stream);
+/* fused_recovery_full_kv, benchmark/rdp/main.py:95-126: the row rebuilt as by
+ * kvec_gs_rdp_recover, and the stream written to kv->k and kv->v.  Same limits. */
+int kvec_gs_rdp_recover_kv(void* shards, const kvec_kv_bhtd* kv, int nd, int S, int star_base, int missing_a,
+                           int missing_b, void* stream);
 /* pack_row_from_block_launcher, bench_ghostserve_rdp.py:152-175:
  * rows[row*S ..] = k_blk words then v_blk words (S >= 2*words). */
 int kvec_gs_pack_row(const void* k_blk, const void* v_blk, void* rows, int64_t words, int row,

@@ -1,0 +1,63 @@
+"""Backup, recovery and encode kernels that read and write K and V where they
+lie, against the oracle on the permuted copies: strided tensors, every row
+count, rows at every alignment, both tile widths, and the layouts that fall
+back to the copies."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _kv(B, H, T, D, order, gpu, seed=0):
+    """K and V indexed [B, H, T, D], random words, in the memory order given."""
+    g = torch.Generator(device="cpu").manual_seed(seed + T)
+    out = []
+    for _ in range(2):
+        x = torch.randint(-32768, 32768, (B, H, T, D), generator=g, dtype=torch.int16)
+        if order == "token":       # [B, T, H, D] cache
+            t = x.permute(0, 2, 1, 3).contiguous().to(gpu).permute(0, 2, 1, 3)
+        elif order == "wide":      # heads of a wider tensor
+            t = torch.zeros((B, H, T, D + 24), dtype=torch.int16, device=gpu)[..., 8:8 + D]
+            t.copy_(x)
+        elif order == "odd":       # two bytes past alignment
+            buf = torch.zeros(x.numel() + 8, dtype=torch.int16, device=gpu)
+            t = buf[1:1 + x.numel()].view(B, H, T, D)
+            t.copy_(x)
+        else:
+            t = x.to(gpu)
+        out.append(t.view(torch.float16))
+    return out
+
+
+def _tn(x):
+    B, H, T, D = x.shape
+    return x.view(torch.int16).permute(2, 0, 1, 3).contiguous().cpu().numpy().reshape(T, -1).view(np.uint16)
+
+
+# nd 1..8 at word counts that leave rows at every alignment; 128-thread tiles
+# (stripes of few tiles) and, for the last three, 512-thread ones; one row
+# that is a whole number of tiles; D of 80 (10 chunks per head)
+@pytest.mark.parametrize("B,H,T,D,nd", [
+    (1, 8, 512, 128, 8), (2, 1, 33, 128, 6), (1, 2, 5, 64, 3), (3, 2, 17, 80, 7), (1, 1, 64, 128, 8),
+    (2, 4, 101, 128, 5), (1, 1, 1024, 8, 4), (1, 3, 7, 16, 2), (4, 8, 263, 128, 1), (4, 8, 521, 128, 2),
+    (8, 8, 800, 128, 6), (1, 2, 4096, 64, 1)])
+@pytest.mark.parametrize("order", ["head", "token", "wide", "odd"])
+def test_gs_rdp_kv_layouts(pkg, ora, gpu, B, H, T, D, nd, order):
+    K, V = _kv(B, H, T, D, order, gpu)
+    sb = (B * T) % 5 - 1
+    want = ora.gs_backup(_tn(K), _tn(V), nd, sb)
+    pk = pkg.rdp.fused_backup_full_kv(K, V, nd, star_base=sb)
+    assert np.array_equal(pk["shards_KV"].cpu().numpy(), want)
+    S = pk["shard_size"]
+    for a, b in [(-1, -1), (nd - 1, -1), (0, -1), (nd // 2, nd)]:
+        sh = want.copy()
+        if 0 <= a < nd:
+            sh[a] = 0x5A5A
+        exp = sh.copy()
+        ora.gs_recover(exp, nd, S, sb, a, b)
+        pk["shards_KV"] = torch.from_numpy(sh.view(np.int16)).to(gpu).view(torch.uint16)
+        k2, v2, _ = pkg.rdp.fused_recovery_full_kv(pk, a, b)
+        assert np.array_equal(pk["shards_KV"].cpu().numpy(), exp), (a, b)
+        assert torch.equal(k2.view(torch.int16), K.view(torch.int16).contiguous()), (a, b)
+        assert torch.equal(v2.view(torch.int16), V.view(torch.int16).contiguous()), (a, b)
