@@ -141,24 +141,30 @@ def forward_encode_kv(keys: torch.Tensor, values: torch.Tensor, num_data_shards:
         pad = num_data_shards * shard_sz - total
     total_shards = num_data_shards + num_parity_shards
     assert shard_sz > 0
-    # K || V and the zero padding go straight into the shard tensor's data rows
-    # (the reference packs into a separate data_padded and the encode copies
-    # it over); the encode then reads the rows in place and writes the parity
-    # rows.  The shard bytes are the same.
     shards = torch.empty((total_shards, shard_sz), dtype=torch.uint16, device=device)
-    data_rows = shards.view(-1)[: num_data_shards * shard_sz]
-    if pad:
-        data_rows.view(torch.int16)[total:].zero_()
-    rs_kernel.pack_fp16_pair_to_u16(keys.contiguous().view(-1), values.contiguous().view(-1),
-                                    data_rows)
-    if scheme == "spec":
-        rows = shards.view(torch.uint8).view(total_shards, -1)
-        spec.rs8_encode([rows[i] for i in range(num_data_shards)],
-                        [rows[num_data_shards + i] for i in range(num_parity_shards)])
-    else:
-        gf_exp, gf_log = device_gf_tables(device)
-        rs_kernel.encode_rs_u16(data_rows, shards, num_data_shards, num_parity_shards, shard_sz,
-                                gf_exp, gf_log)
+    keys = keys.contiguous()
+    values = values.contiguous()
+    # one pass over K and V for the rows and the parity, when the layout allows it
+    if not (scheme == "ghostserve" and N_k == N_v and
+            _lib.call_if_built("kvec_rs16_encode_kv", keys.data_ptr(), values.data_ptr(), 2 * N_k,
+                               shards.data_ptr(), int(num_data_shards), int(num_parity_shards),
+                               int(shard_sz), _stream(shards))):
+        # K || V and the zero padding go straight into the shard tensor's data
+        # rows (the reference packs into a separate data_padded and the encode
+        # copies it over); the encode then reads the rows in place and writes
+        # the parity rows.  The shard bytes are the same.
+        data_rows = shards.view(-1)[: num_data_shards * shard_sz]
+        if pad:
+            data_rows.view(torch.int16)[total:].zero_()
+        rs_kernel.pack_fp16_pair_to_u16(keys.view(-1), values.view(-1), data_rows)
+        if scheme == "spec":
+            rows = shards.view(torch.uint8).view(total_shards, -1)
+            spec.rs8_encode([rows[i] for i in range(num_data_shards)],
+                            [rows[num_data_shards + i] for i in range(num_parity_shards)])
+        else:
+            gf_exp, gf_log = device_gf_tables(device)
+            rs_kernel.encode_rs_u16(data_rows, shards, num_data_shards, num_parity_shards,
+                                    shard_sz, gf_exp, gf_log)
     meta = {
         "B": B, "H": H, "T": T, "D": D,
         "N_k": N_k, "N_v": N_v,

@@ -320,6 +320,14 @@ int kvec_rs16_split(const void* in, void* k_out, void* v_out, int64_t N_k, int64
 int kvec_rs16_encode(const void* data_padded, void* shards, int data_shards, int parity_shards,
                      int shard_size, const uint16_t* gf_exp, const uint16_t* gf_log,
                      void* stream);
+/* forward_encode_kv, benchmark/rs/main.py:63-137, in one pass: the data rows
+ * are K || V || zeros (kv_half_bytes raw bytes each) and the parity rows those
+ * of kvec_rs16_encode with the tables of kvec_gf16_tables.  Every byte of
+ * shards is written.  KVEC_EUNSUPPORTED, with nothing enqueued, outside: 1 to 4
+ * parity rows, K, V, shards and kv_half_bytes multiples of 16, shard_size >=
+ * 64, K and V below 1 GiB, shards below 2 GiB. */
+int kvec_rs16_encode_kv(const void* key_input, const void* value_input, int64_t kv_half_bytes, void* shards,
+                        int data_shards, int parity_shards, int shard_size, void* stream);
 /* reconstruct_rs_u16_inplace, :287-312: rebuild the m data rows listed in the
  * device int32 array missing_data from the parity rows in parity_used (device,
  * m entries; m <= 16 as the reference's, any data_shards >= m).  Parity rows

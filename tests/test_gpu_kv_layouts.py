@@ -61,3 +61,21 @@ def test_gs_rdp_kv_layouts(pkg, ora, gpu, B, H, T, D, nd, order):
         assert np.array_equal(pk["shards_KV"].cpu().numpy(), exp), (a, b)
         assert torch.equal(k2.view(torch.int16), K.view(torch.int16).contiguous()), (a, b)
         assert torch.equal(v2.view(torch.int16), V.view(torch.int16).contiguous()), (a, b)
+
+
+# (k, m) with one to four parities (packed words and bit planes; five takes the
+# pack and the general encode), rows of multiples of 16 bytes and not, odd and
+# even k, rows under a tile, a whole number of tiles, tiles and 2-30 bytes,
+# zero padding across several rows, stripes of many tiles
+@pytest.mark.parametrize("k,m", [(4, 1), (5, 2), (6, 2), (1, 1), (5, 3), (8, 3), (10, 4), (16, 4), (3, 4), (17, 2),
+                                 (6, 5)])
+@pytest.mark.parametrize("B,H,T,D", [(1, 1, 40, 16), (1, 2, 33, 128), (2, 3, 101, 80), (1, 8, 256, 128),
+                                     (1, 1, 2051, 8), (3, 4, 521, 128)])
+def test_rs16_encode_kv(pkg, ora, gpu, k, m, B, H, T, D):
+    K, V = _kv(B, H, T, D, "head", gpu, seed=k)
+    sh, meta = pkg.rs.forward_encode_kv(K, V, k, m)
+    S = meta["shard_sz"]
+    data = np.zeros(k * S, np.uint16)
+    flat = np.concatenate([x.view(torch.int16).cpu().numpy().reshape(-1).view(np.uint16) for x in (K, V)])
+    data[:flat.size] = flat
+    assert np.array_equal(sh.cpu().numpy(), ora.rs16_encode(data, k, m, S, *pkg.rs.init_gf_tables()))
