@@ -116,6 +116,7 @@ SIGNATURES = {
     "kvec_rs16_split": (_i, [_vp, _vp, _vp, _i64, _i64, _vp]),
     "kvec_rs16_encode": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp, _vp]),
     "kvec_rs16_encode_kv": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i, _vp]),
+    "kvec_rs16_recover_kv": (_i, [_vp, _vp, _vp, _i64, _i, _i, _i, _vp, _i, _vp]),
     "kvec_rs16_reconstruct": (_i, [_vp, _i, _i, _i, _vp, _i, _vp, _vp, _vp, _vp]),
     "kvec_gf16_tables": (_i, [_vp, _vp]),
 }

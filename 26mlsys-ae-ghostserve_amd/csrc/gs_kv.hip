@@ -143,9 +143,6 @@ __global__ __launch_bounds__(BS) void gs_recover_kv_kernel(uint8_t* sh, uint32_t
         e1[i] = chunk_load(rs, live && lane == 63 && m ? my + 16 : kNoLoad);
     }
     __builtin_amdgcn_sched_barrier(0);
-    auto put_byte = [&](uint32_t x, uint8_t b) {
-        if (x < out_len) *as_global(kv_at<FLAT>(dst, x)) = b;
-    };
     u32x4 acc = {0, 0, 0, 0};
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
@@ -157,34 +154,15 @@ __global__ __launch_bounds__(BS) void gs_recover_kv_kernel(uint8_t* sh, uint32_t
     }
     if (blockIdx.x == 0) {
         for (uint32_t u = threadIdx.x; u < 32 * ND; u += BS) {
-            const uint32_t j = uint32_t(row_of(int(u >> 5))), b = u & 31;
-            const uint32_t r0 = j * Sb, r1 = r0 + Sb, first = (r0 + 15) & ~15u;
-            const uint32_t x = b < 16 ? r0 + b : (r1 & ~15u) + (b - 16);
-            const bool mine = b < 16 ? x < first && x < r1 : x >= first && x < r1;
-            if (j < uint32_t(ND) && mine) put_byte(x, as_global(sh)[x]);
+            const uint32_t j = uint32_t(row_of(int(u >> 5)));
+            if (j < uint32_t(ND)) kv_put_row_end<FLAT>(dst, sh, Sb, j, u & 31);
         }
     }
     if (t < 0) return;
     *reinterpret_cast<u32x4*>(tile + 16 * threadIdx.x) = acc;
     __syncthreads();
     tile_store<false, BS>(sh + uint32_t(t) * Sb + t0, tile, nbytes);
-    // the same bytes to K and V
-    const uint32_t D0 = uint32_t(t) * Sb + t0, E = D0 + nbytes;
-    const uint32_t A0 = (D0 + 15) & ~15u, A1 = E & ~15u;
-    if (A0 < A1) {
-        const uint32_t sh0 = A0 - D0;   // < 16
-        for (uint32_t k = threadIdx.x; k < (A1 - A0) >> 4; k += BS) {
-            u32x4 v = *reinterpret_cast<const u32x4*>(tile + 16 * k);
-            if (sh0) v = funnel16(v, *reinterpret_cast<const u32x4*>(tile + 16 * k + 16), sh0);
-            const uint32_t X = A0 + 16 * k;
-            if (X + 16 <= out_len) st_stream(kv_at<FLAT>(dst, X), 0, v);
-        }
-        const uint32_t i = threadIdx.x;
-        if (i < 16 && D0 + i < A0) put_byte(D0 + i, tile[i]);
-        else if (i >= 16 && i < 32 && A1 + (i - 16) < E) put_byte(A1 + (i - 16), tile[A1 + (i - 16) - D0]);
-    } else {
-        for (uint32_t x = D0 + threadIdx.x; x < E; x += BS) put_byte(x, tile[x - D0]);
-    }
+    kv_put_tile<FLAT, BS>(dst, tile, uint32_t(t) * Sb + t0, nbytes);
 }
 
 // ---------------------------------------------------------------- host side

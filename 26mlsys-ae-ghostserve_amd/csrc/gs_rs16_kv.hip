@@ -11,7 +11,7 @@
 //
 // A wave owns NW KiB of every row and walks the rows from the last to the
 // first (Horner's rule: parity p = (...(D_{k-1} g + D_{k-2}) g + ...) g + D_0,
-// g = 2^(p+1)), each row's chunks loaded two rows ahead.
+// g = 2^(p+1)), each row's chunks loaded two or four rows ahead.
 //
 // Products.  With one or two outputs the accumulators hold packed words and
 // are doubled in place (gf16.h, about 5 VALU operations per two doublings of
@@ -133,6 +133,7 @@ struct RsAcc<M, 4, true> {
     __device__ __forceinline__ void shift() {
         if constexpr (P < M) {
             plane_step<P + 1, false>(a[P], a[P]);
+            pin(a[P]);
             shift<P + 1>();
         }
     }
@@ -148,6 +149,10 @@ struct RsAcc<M, 4, true> {
     __device__ __forceinline__ void finish() {
 #pragma unroll
         for (int p = 0; p < M; ++p) to_planes(a[p]);
+    }
+    // after finish()
+    __device__ __forceinline__ void add_window(int p, int n, u32x4 v) {
+        a[p][4 * n] ^= v.x, a[p][4 * n + 1] ^= v.y, a[p][4 * n + 2] ^= v.z, a[p][4 * n + 3] ^= v.w;
     }
     __device__ __forceinline__ u32x4 window(int p, int n) const {
         return u32x4{a[p][4 * n], a[p][4 * n + 1], a[p][4 * n + 2], a[p][4 * n + 3]};
@@ -180,6 +185,9 @@ struct RsAcc<M, NW, false> {
     __device__ __forceinline__ void fold(const u32x4 (&x)[NW]) { step(x); }
     __device__ __forceinline__ void shift() { step(nullptr); }
     __device__ __forceinline__ void finish() {}
+    __device__ __forceinline__ void add_window(int p, int n, u32x4 v) {
+        a[p][n][0] ^= v.x, a[p][n][1] ^= v.y, a[p][n][2] ^= v.z, a[p][n][3] ^= v.w;
+    }
     __device__ __forceinline__ u32x4 window(int p, int n) const {
         return u32x4{a[p][n][0], a[p][n][1], a[p][n][2], a[p][n][3]};
     }
@@ -277,12 +285,20 @@ __global__ __launch_bounds__(BS) void rs16_encode_kv_kernel(KvStream src, uint8_
         const uint32_t X = (data_end & ~15u) + 2 * threadIdx.x;
         if (X < data_end) *as_global(reinterpret_cast<uint16_t*>(sh + X)) = KvReader<true>(src).word(X);
     }
-    // Two sets, the loop unrolled by two so that none is copied; an odd k gets
-    // a row of zeros above the last, which leaves the accumulators zero.
+    // Two sets, the loop unrolled by two so that none is copied; the last row
+    // of an odd k comes before it (a skip inside cost 16 % in copies).
     RowChunks<NW, ALIGNED> ra, rb;
-    int i = (k - 1) | 1;
-    load(i, ra);
-    load(i - 1, rb);
+    int i = k - 1;
+    if (k & 1) {
+        load(i, rb);
+        load(i - 1, ra);
+        use(i, rb);
+        load(i - 2, rb);
+        --i;
+    } else {
+        load(i, ra);
+        load(i - 1, rb);
+    }
     for (; i > 0; i -= 2) {
         use(i, ra);
         load(i - 2, ra);
@@ -305,6 +321,142 @@ __global__ __launch_bounds__(BS) void rs16_encode_kv_kernel(KvStream src, uint8_
     for (int p = 0; p < M; ++p) tile_store<true, BS>(par + uint32_t(p) * Sb, tile[p], nbytes);
 }
 
+// ------------------------------------------------------------------- decode
+// M lost data rows of a shard tensor sh from the surviving rows and parity
+// rows 0 .. M-1: syndrome r is b_r = Par_r ^ XOR_j D_j 2^((r+1) j) over the
+// surviving rows, by Horner's rule over all k rows with a lost row adding
+// nothing, and the lost rows are x_c = XOR_r inv[c][r] b_r through byte maps
+// (gf16.h) that the host built and each block stages in LDS.  The surviving
+// rows' whole chunks go to K and V from the registers they were loaded into,
+// their ends byte by byte from block 0, the rebuilt rows to their place in sh
+// and to K and V.
+// Measured (kernel trace, fresh outputs): two of six rows lost, 16 x 8 x 2048
+// x 128 bf16, 57 us for 313 MB (5.5 TB/s); 4 x 8 x 1001 x 128 13.7 us for 38 MB,
+// where the reconstruct and the copies took 19 us beside two blocking uploads
+// of the indices (whole call 60 -> 14 us).
+template <int M>
+struct RsRec {
+    uint64_t lost;        // data rows, bit i
+    uint32_t row[M];      // the lost rows, in order
+    uint32_t maps[M * M][kRs16Tab];
+};
+
+template <int M, int NW, int R, bool PLANES, int BS, bool ALIGNED>
+__global__ __launch_bounds__(BS) void rs16_recover_kv_kernel(KvStream dst, uint8_t* sh, uint32_t sh_bytes, uint32_t Sb,
+                                                             int k, RsRec<M> rec) {
+    constexpr uint32_t TB = 16 * BS * NW, WB = 1024 * NW;
+    __shared__ __attribute__((aligned(16))) uint8_t tile[ALIGNED ? 1 : M][ALIGNED ? 16 : TB + 16];
+    __shared__ __attribute__((aligned(16))) uint32_t maps[M * M][kRs16Tab];
+    for (uint32_t e = threadIdx.x; e < M * M * kRs16Tab; e += BS) maps[e / kRs16Tab][e % kRs16Tab] = rec.maps[e / kRs16Tab][e % kRs16Tab];
+    const uint32_t t0 = blockIdx.x * TB;
+    const uint32_t nbytes = Sb - t0 < TB ? Sb - t0 : TB;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wb = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))) * WB;
+    const uint32_t kb = dst.kb;
+    const __amdgpu_buffer_rsrc_t rs = chunk_rsrc(sh, (sh_bytes + 15) & ~15u);
+    auto absent = [&](int i) { return i >= k || ((rec.lost >> (i & 63)) & 1); };   // i >= 0
+    auto at = [&](int i) { return uint32_t(i >= 0 ? i : k - 1 - i) * Sb + t0 + wb; };
+    // row i, or parity row -1 - i
+    auto load = [&](int i, RowChunks<NW, ALIGNED>& s) {
+        if (i < -M || (i >= 0 && absent(i))) return;   // uniform
+        const uint32_t A = at(i), m = ALIGNED ? 0 : A & 15, x = A - m;
+#pragma unroll
+        for (int n = 0; n < NW; ++n) s.c[n] = chunk_load(rs, x + n * 1024 + 16 * lane);
+        if (!ALIGNED) s.e = chunk_load(rs, x + WB);
+    };
+    RsAcc<M, NW, PLANES> acc;
+    acc.clear();
+    auto use = [&](int i, const RowChunks<NW, ALIGNED>& s) {
+        if (!PLANES && i >= k) return;   // the accumulators are still zero
+        if (absent(i)) {
+            acc.shift();
+            return;
+        }
+        const uint32_t A = at(i), m = ALIGNED ? 0 : A & 15, x = A - m, r0 = uint32_t(i) * Sb, rend = r0 + Sb;
+        if (x >= r0 && x + WB <= rend && (x + WB <= kb || (x >= kb && x + WB <= 2 * kb))) {   // uniform
+            uint8_t* p = x >= kb ? dst.V + (x - kb) : dst.K + x;
+#pragma unroll
+            for (int n = 0; n < NW; ++n) st_stream(p + n * 1024, 16 * lane, s.c[n]);
+        } else {
+#pragma unroll
+            for (int n = 0; n < NW; ++n) {
+                const uint32_t X = x + n * 1024 + 16 * lane;
+                if (X >= r0 && X + 16 <= rend && X < 2 * kb) st_stream(kv_at<true>(dst, X), 0, s.c[n]);
+            }
+        }
+        u32x4 w[NW];
+        s.windows(m, w);
+        acc.fold(w);
+    };
+    if (!ALIGNED && blockIdx.x == 0)
+        for (uint32_t u = threadIdx.x; u < 32 * uint32_t(k); u += BS)
+            if (!absent(int(u >> 5))) kv_put_row_end<true>(dst, sh, Sb, u >> 5, u & 31);
+    RowChunks<NW, ALIGNED> row[R];
+    int i = (k + R - 1) / R * R - 1;
+#pragma unroll
+    for (int j = 0; j < R; ++j) load(i - j, row[j]);
+    for (; i >= 0; i -= R) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            use(i - j, row[j]);
+            load(i - j - R, row[j]);
+        }
+    }
+    // row[r] holds parity row r
+    acc.finish();
+#pragma unroll
+    for (int r = 0; r < M; ++r) {
+        u32x4 w[NW];
+        row[r % R].windows(ALIGNED ? 0 : at(-1 - r) & 15, w);
+#pragma unroll
+        for (int n = 0; n < NW; ++n) acc.add_window(r, n, w[n]);
+        if (r + R < M) load(-1 - r - R, row[r % R]);
+    }
+    __syncthreads();   // maps
+#pragma unroll
+    for (int n = 0; n < NW; ++n) {
+        Gf8Fields f[M][4];
+#pragma unroll
+        for (int r = 0; r < M; ++r) {
+            uint32_t by[4];
+            split_bytes(acc.window(r, n), by);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) f[r][q] = gf8_fields(by[q]);
+        }
+        const uint32_t o = wb + n * 1024 + 16 * lane;
+#pragma unroll
+        for (int c = 0; c < M; ++c) {
+            uint32_t v[4] = {0, 0, 0, 0};
+#pragma unroll
+            for (int r = 0; r < M; ++r) {
+                const uint32_t* T = maps[c * M + r];
+                v[0] = gf16_fma2(v[0], f[r][0], T + 0, f[r][1], T + 6);
+                v[1] = gf16_fma2(v[1], f[r][0], T + 12, f[r][1], T + 18);
+                v[2] = gf16_fma2(v[2], f[r][2], T + 0, f[r][3], T + 6);
+                v[3] = gf16_fma2(v[3], f[r][2], T + 12, f[r][3], T + 18);
+                // one coefficient's maps live at a time
+                asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]) :: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            const u32x4 x = join_bytes(v);
+            if (!ALIGNED) {
+                *reinterpret_cast<u32x4*>(tile[c] + o) = x;
+            } else if (o < nbytes) {
+                const uint32_t X = rec.row[c] * Sb + t0 + o;
+                st_stream(sh, X, x);
+                if (X < 2 * kb) st_stream(kv_at<true>(dst, X), 0, x);
+            }
+        }
+    }
+    if (ALIGNED) return;
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < M; ++c) {
+        tile_store<false, BS>(sh + rec.row[c] * Sb + t0, tile[c], nbytes);
+        kv_put_tile<true, BS>(dst, tile[c], rec.row[c] * Sb + t0, nbytes);
+    }
+}
+
 // ---------------------------------------------------------------- host side
 typedef void (*RsEncKvFn)(KvStream, uint8_t*, uint32_t, int);
 struct RsKvKern {
@@ -320,6 +472,107 @@ static RsKvKern rs_encode_kv(int m) {
         case 3: return {&rs16_encode_kv_kernel<3, 4, true, 256, ALIGNED>, 256, 4};
         case 4: return {&rs16_encode_kv_kernel<4, 4, true, 256, ALIGNED>, 256, 4};
         default: return {nullptr, 0, 0};
+    }
+}
+
+// ------------------------------------------------ the inverse, on the host
+struct Gf16Tables {
+    uint16_t ex[2 * 65535], lg[65536];
+    Gf16Tables() { kvec_gf16_tables(ex, lg); }
+    uint16_t mul(uint16_t a, uint16_t b) const { return a && b ? ex[uint32_t(lg[a]) + lg[b]] : uint16_t(0); }
+    uint16_t inv(uint16_t a) const { return ex[65535 - lg[a]]; }   // a != 0
+};
+
+static const Gf16Tables& gf16_tables() {
+    static const Gf16Tables t;
+    return t;
+}
+
+// Inverse of V[r][c] = 2^((r + 1) row[c]) by the reference's Gauss-Jordan
+// (benchmark/rs/kernel.cu:135-185: pivot order, a zero column skipped).
+template <int M>
+static void rs_inverse(const uint32_t* row, uint16_t (&inv)[M][M]) {
+    const Gf16Tables& g = gf16_tables();
+    uint16_t V[M][M];
+    for (int r = 0; r < M; ++r)
+        for (int c = 0; c < M; ++c) {
+            V[r][c] = g.ex[(uint32_t(r + 1) * row[c]) % 65535];
+            inv[r][c] = r == c;
+        }
+    for (int i = 0; i < M; ++i) {
+        int pr = i;
+        while (pr < M && V[pr][i] == 0) ++pr;
+        if (pr == M) continue;
+        for (int c = 0; c < M && pr != i; ++c) {
+            uint16_t t = V[i][c];
+            V[i][c] = V[pr][c], V[pr][c] = t;
+            t = inv[i][c];
+            inv[i][c] = inv[pr][c], inv[pr][c] = t;
+        }
+        const uint16_t ip = g.inv(V[i][i]);
+        for (int c = 0; c < M; ++c) {
+            V[i][c] = g.mul(V[i][c], ip);
+            inv[i][c] = g.mul(inv[i][c], ip);
+        }
+        for (int r = 0; r < M; ++r) {
+            const uint16_t f = V[r][i];
+            if (r == i || !f) continue;
+            for (int c = 0; c < M; ++c) {
+                V[r][c] ^= g.mul(f, V[i][c]);
+                inv[r][c] ^= g.mul(f, inv[i][c]);
+            }
+        }
+    }
+}
+
+// The byte maps of coefficient c in the order gf16_fma2 reads them: low to
+// low, high to low, low to high, high to high byte; two dwords per 3-bit field.
+static void byte_maps(uint16_t c, uint32_t (&out)[kRs16Tab]) {
+    const Gf16Tables& g = gf16_tables();
+    for (int d = 0; d < kRs16Tab; ++d) {
+        const int src = (d / 6) & 1, dst = d / 12, f = (d % 6) >> 1, half = d & 1;
+        uint32_t dw = 0;
+        for (int q = 0; q < 4; ++q) {
+            const int v = half * 4 + q;
+            if (f == 2 && v >= 4) continue;
+            const uint16_t y = g.mul(uint16_t((v << (3 * f)) << (8 * src)), c);
+            dw |= uint32_t((y >> (8 * dst)) & 0xFF) << (8 * q);
+        }
+        out[d] = dw;
+    }
+}
+
+// One or two lost rows: 256 threads with four rows in flight, or 512 with two
+// from 8 MiB rows on (kernel trace, RS(6, 2), two rows lost: 5.5 MB rows 13.7
+// us either way, 0.7 MB 8.8 against 9.2; whole calls with 22 MB rows 57 against
+// 59-61 us).  More: bit planes, two rows of four windows in flight; 128 and 512
+// threads ran 39 and 43 against 35 us (16 rows of 4.2 MB, four lost).
+template <int M>
+static void rs_recover_launch(KvStream dst, uint8_t* sh, uint64_t sh_bytes, uint32_t Sb, int k, const int32_t* missing,
+                              hipStream_t st) {
+    RsRec<M> rec{};
+    for (int c = 0; c < M; ++c) {
+        rec.row[c] = uint32_t(missing[c]);
+        rec.lost |= uint64_t(1) << missing[c];
+    }
+    uint16_t inv[M][M];
+    rs_inverse<M>(rec.row, inv);
+    for (int c = 0; c < M; ++c)
+        for (int r = 0; r < M; ++r) byte_maps(inv[c][r], rec.maps[c * M + r]);
+    auto launch = [&](auto kern, int bs, int nw) {
+        hipLaunchKernelGGL(kern, dim3(blocks_for(int64_t(Sb), 16 * bs * nw)), dim3(bs), 0, st, dst, sh,
+                           uint32_t(sh_bytes), Sb, k, rec);
+    };
+    const bool aligned = Sb % 16 == 0;
+    if constexpr (M > 2) {
+        if (aligned) launch(&rs16_recover_kv_kernel<M, 4, 2, true, 256, true>, 256, 4);
+        else launch(&rs16_recover_kv_kernel<M, 4, 2, true, 256, false>, 256, 4);
+    } else if (Sb < (8u << 20)) {
+        if (aligned) launch(&rs16_recover_kv_kernel<M, 1, 4, false, 256, true>, 256, 1);
+        else launch(&rs16_recover_kv_kernel<M, 1, 4, false, 256, false>, 256, 1);
+    } else {
+        if (aligned) launch(&rs16_recover_kv_kernel<M, 1, 2, false, 512, true>, 512, 1);
+        else launch(&rs16_recover_kv_kernel<M, 1, 2, false, 512, false>, 512, 1);
     }
 }
 
@@ -347,5 +600,38 @@ extern "C" int kvec_rs16_encode_kv(const void* key_input, const void* value_inpu
     if (int rc = check_no_alias(&w, 1, r, 2, fn)) return rc;
     hipLaunchKernelGGL(kern.fn, dim3(blocks_for(int64_t(Sb), 16 * kern.bs * kern.nw)), dim3(kern.bs), 0,
                        as_stream(stream), s, (uint8_t*)shards, uint32_t(Sb), data_shards);
+    return check_launch(fn);
+}
+
+extern "C" int kvec_rs16_recover_kv(void* shards, void* key_output, void* value_output, int64_t kv_half_bytes,
+                                    int data_shards, int parity_shards, int shard_size, const int32_t* missing,
+                                    int n_missing, void* stream) {
+    static const char* fn = "kvec_rs16_recover_kv";
+    if (!shards || (n_missing > 0 && !missing)) return set_error(KVEC_EINVAL, "%s: null pointer", fn);
+    if (n_missing > 0 && n_missing > parity_shards)
+        return set_error(KVEC_EINVAL, "%s: %d lost rows, %d parity rows", fn, n_missing, parity_shards);
+    for (int q = 0; q < n_missing; ++q)
+        if (missing[q] < 0 || missing[q] >= data_shards || (q && missing[q] <= missing[q - 1]))
+            return set_error(KVEC_EINVAL, "%s: lost rows must be ascending data rows", fn);
+    KvStream s{};
+    bool flat = false;
+    const uint64_t Sb = uint64_t(shard_size > 0 ? shard_size : 0) * 2;
+    const uint64_t bytes = Sb * (uint64_t(data_shards > 0 ? data_shards : 0) + uint64_t(parity_shards > 0 ? parity_shards : 0));
+    if (n_missing < 1 || n_missing > 4 || data_shards < 1 || data_shards > 64 || parity_shards > 65535 ||
+        shard_size < 64 || !aligned16(shards) || bytes > (uint64_t(1) << 31) - 16 || kv_half_bytes < 16 ||
+        !make_kv_stream(&s, &flat, key_output, value_output, KvDims{1, 1, 1, kv_half_bytes, 0, 0, 0}) ||
+        2 * uint64_t(s.kb) > uint64_t(data_shards) * Sb)
+        return set_error(KVEC_EUNSUPPORTED, "%s: layout or stripe not built", fn);
+    if (!key_output || !value_output) return set_error(KVEC_EINVAL, "%s: null K or V", fn);
+    const Span w[3] = {{shards, bytes, "shards", -1}, {key_output, s.kb, "K", -1}, {value_output, s.kb, "V", -1}};
+    if (int rc = check_no_alias(w, 3, nullptr, 0, fn)) return rc;
+    uint8_t* sh = (uint8_t*)shards;
+    const hipStream_t st = as_stream(stream);
+    switch (n_missing) {
+        case 1: rs_recover_launch<1>(s, sh, bytes, uint32_t(Sb), data_shards, missing, st); break;
+        case 2: rs_recover_launch<2>(s, sh, bytes, uint32_t(Sb), data_shards, missing, st); break;
+        case 3: rs_recover_launch<3>(s, sh, bytes, uint32_t(Sb), data_shards, missing, st); break;
+        default: rs_recover_launch<4>(s, sh, bytes, uint32_t(Sb), data_shards, missing, st); break;
+    }
     return check_launch(fn);
 }

@@ -76,6 +76,48 @@ __device__ __forceinline__ uint8_t* kv_at(const KvStream& s, uint32_t x) {
     return (in_v ? s.V : s.K) + kv_off<FLAT>(s, in_v ? x - s.kb : x);
 }
 
+// The byte at stream position x, dropped past V's end.
+template <bool FLAT>
+__device__ __forceinline__ void kv_put_byte(const KvStream& s, uint32_t x, uint8_t b) {
+    if (x < 2 * s.kb) *as_global(kv_at<FLAT>(s, x)) = b;
+}
+
+// Bytes of packed row j (Sb bytes each, at sh) that no whole aligned chunk of
+// the row holds, b in [0, 32): the at most 15 before the first (b < 16) and
+// after the last, copied to K or V.
+template <bool FLAT>
+__device__ __forceinline__ void kv_put_row_end(const KvStream& s, const uint8_t* sh, uint32_t Sb, uint32_t j,
+                                               uint32_t b) {
+    const uint32_t r0 = j * Sb, r1 = r0 + Sb, first = (r0 + 15) & ~15u;
+    const uint32_t x = b < 16 ? r0 + b : (r1 & ~15u) + (b - 16);
+    if (b < 16 ? x < first && x < r1 : x >= first && x < r1) kv_put_byte<FLAT>(s, x, as_global(sh)[x]);
+}
+
+// Stream bytes [D0, D0 + nbytes) from the LDS tile (16 bytes of slack) to K
+// and V: whole chunks, then the bytes around them.  All BS threads call it.
+template <bool FLAT, int BS>
+__device__ __forceinline__ void kv_put_tile(const KvStream& s, const uint8_t* tile, uint32_t D0, uint32_t nbytes) {
+    const uint32_t out_len = 2 * s.kb;
+    const uint32_t E = D0 + nbytes, A0 = (D0 + 15) & ~15u, A1 = E & ~15u;
+    auto put_byte = [&](uint32_t x, uint8_t b) {
+        if (x < out_len) *as_global(kv_at<FLAT>(s, x)) = b;
+    };
+    if (A0 < A1) {
+        const uint32_t m = A0 - D0;   // < 16
+        for (uint32_t k = threadIdx.x; k < (A1 - A0) >> 4; k += BS) {
+            u32x4 v = *reinterpret_cast<const u32x4*>(tile + 16 * k);
+            if (m) v = funnel16(v, *reinterpret_cast<const u32x4*>(tile + 16 * k + 16), m);
+            const uint32_t X = A0 + 16 * k;
+            if (X + 16 <= out_len) st_stream(kv_at<FLAT>(s, X), 0, v);
+        }
+        const uint32_t i = threadIdx.x;
+        if (i < 16 && D0 + i < A0) put_byte(D0 + i, tile[i]);
+        else if (i >= 16 && i < 32 && A1 + (i - 16) < E) put_byte(A1 + (i - 16), tile[A1 + (i - 16) - D0]);
+    } else {
+        for (uint32_t x = D0 + threadIdx.x; x < E; x += BS) put_byte(x, tile[x - D0]);
+    }
+}
+
 // Host: the stream of K and V indexed [B][H][T][D] with the given byte
 // strides.  *flat is set when the token-major order is memory order.  False
 // when the layout is not one these kernels take.

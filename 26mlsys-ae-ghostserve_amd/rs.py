@@ -208,10 +208,25 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
             spec.rs8_decode([rows[i] for i in range(num_data + num_parity)], num_data,
                             [int(i) for i in missing_shards])
         missing_data = []
-    gf_exp, gf_log = device_gf_tables(device)
+    dtype = meta.get("dtype", torch.float16)
+    N_k, N_v = meta["N_k"], meta["N_v"]
+    B, H, T, D = meta["B"], meta["H"], meta["T"], meta["D"]
+    K = torch.empty(N_k, dtype=dtype, device=device)
+    V = torch.empty(N_v, dtype=dtype, device=device)
+    # the rebuild and the split in one pass when the first parity rows serve
+    # and the layout allows it
+    if (missing_data and N_k == N_v and avail_par[:len(missing_data)] == list(range(len(missing_data)))
+            and shards.is_cuda and shards.is_contiguous()
+            and K.element_size() == 2 and shards.element_size() == 2):
+        lost = np.asarray(missing_data, dtype=np.int32)
+        if _lib.call_if_built("kvec_rs16_recover_kv", shards.data_ptr(), K.data_ptr(), V.data_ptr(),
+                              2 * int(N_k), int(num_data), int(num_parity), int(shard_sz),
+                              lost.ctypes.data, len(missing_data), _stream(shards)):
+            return K.view(B, H, T, D), V.view(B, H, T, D)
     if missing_data:
         if len(missing_data) > 16:
             raise RuntimeError("Reconstruction supports at most 16 missing data shards at once.")
+        gf_exp, gf_log = device_gf_tables(device)
         missing_data_t = torch.tensor(missing_data, dtype=torch.int32, device=device)
         parity_used_t = torch.tensor(avail_par[:len(missing_data)], dtype=torch.int32,
                                      device=device)
@@ -219,9 +234,5 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
                                              missing_data_t, parity_used_t, gf_exp, gf_log)
 
     data_area = shards[:num_data].contiguous().view(-1)[:meta["total"]]
-    dtype = meta.get("dtype", torch.float16)
-    K = torch.empty(meta["N_k"], dtype=dtype, device=device)
-    V = torch.empty(meta["N_v"], dtype=dtype, device=device)
-    rs_kernel.u16_to_fp16_split(data_area, K, V, meta["N_k"], meta["N_v"])
-    B, H, T, D = meta["B"], meta["H"], meta["T"], meta["D"]
+    rs_kernel.u16_to_fp16_split(data_area, K, V, N_k, N_v)
     return K.view(B, H, T, D), V.view(B, H, T, D)

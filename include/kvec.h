@@ -336,6 +336,15 @@ int kvec_rs16_encode_kv(const void* key_input, const void* value_input, int64_t 
 int kvec_rs16_reconstruct(void* shards, int shard_size, int data_shards, int parity_shards,
                           const int32_t* missing_data, int m, const int32_t* parity_used,
                           const uint16_t* gf_exp, const uint16_t* gf_log, void* stream);
+/* backwards_decode_kv, benchmark/rs/main.py:140-206, in one pass: the lost data
+ * rows (host int32 array, ascending) rebuilt in place from the surviving rows
+ * and parity rows 0 .. n_missing-1 with the tables of kvec_gf16_tables, and the
+ * rows' first 2*kv_half_bytes bytes written to K and V.  KVEC_EUNSUPPORTED, with
+ * nothing enqueued, outside: 1 to 4 lost rows, data_shards <= 64, and the
+ * limits of kvec_rs16_encode_kv. */
+int kvec_rs16_recover_kv(void* shards, void* key_output, void* value_output, int64_t kv_half_bytes,
+                         int data_shards, int parity_shards, int shard_size, const int32_t* missing, int n_missing,
+                         void* stream);
 /* init_gf_tables, benchmark/rs/main.py:39-54, into host arrays (exp: 131070
  * entries, log: 65536). */
 int kvec_gf16_tables(uint16_t* gf_exp, uint16_t* gf_log);

@@ -71,11 +71,37 @@ def test_gs_rdp_kv_layouts(pkg, ora, gpu, B, H, T, D, nd, order):
                                  (6, 5)])
 @pytest.mark.parametrize("B,H,T,D", [(1, 1, 40, 16), (1, 2, 33, 128), (2, 3, 101, 80), (1, 8, 256, 128),
                                      (1, 1, 2051, 8), (3, 4, 521, 128)])
-def test_rs16_encode_kv(pkg, ora, gpu, k, m, B, H, T, D):
+def test_rs16_kv(pkg, ora, gpu, k, m, B, H, T, D):
+    _rs16_round(pkg, ora, gpu, k, m, B, H, T, D)
+
+
+# rows past 8 MiB, the other tile width of the decode
+@pytest.mark.parametrize("k,m,T", [(2, 2, 8193), (1, 1, 4098), (3, 2, 12289)])
+def test_rs16_kv_long_rows(pkg, ora, gpu, k, m, T):
+    _rs16_round(pkg, ora, gpu, k, m, 1, 4, T, 128)
+
+
+def _rs16_round(pkg, ora, gpu, k, m, B, H, T, D):
     K, V = _kv(B, H, T, D, "head", gpu, seed=k)
     sh, meta = pkg.rs.forward_encode_kv(K, V, k, m)
     S = meta["shard_sz"]
     data = np.zeros(k * S, np.uint16)
     flat = np.concatenate([x.view(torch.int16).cpu().numpy().reshape(-1).view(np.uint16) for x in (K, V)])
     data[:flat.size] = flat
-    assert np.array_equal(sh.cpu().numpy(), ora.rs16_encode(data, k, m, S, *pkg.rs.init_gf_tables()))
+    want = ora.rs16_encode(data, k, m, S, *pkg.rs.init_gf_tables())
+    assert np.array_equal(sh.cpu().numpy(), want)
+    # one to m lost rows, at both ends and adjacent; a lost parity row 0 (the
+    # general reconstruct); every byte of the shards as encoded afterwards
+    lost = [list(range(n)) for n in range(1, min(m, k) + 1)] + [list(range(k - n, k)) for n in range(1, min(m, k) + 1)]
+    lost += [[0, k - 1], [k // 2]] if m > 1 and k > 1 else []
+    lost += [[k // 2, k]] if m > 1 else []
+    full = sh.clone()
+    for er in lost:
+        sh.copy_(full)
+        for e in er:
+            if e < k:
+                sh.view(torch.int16)[e] = 0x5A5A
+        k2, v2 = pkg.rs.backwards_decode_kv(sh, meta, er)
+        assert torch.equal(sh.view(torch.int16), full.view(torch.int16)), er
+        assert torch.equal(k2.view(torch.int16), K.view(torch.int16)), er
+        assert torch.equal(v2.view(torch.int16), V.view(torch.int16)), er
