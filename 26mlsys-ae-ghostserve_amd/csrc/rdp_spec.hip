@@ -13,9 +13,8 @@
 //
 // Decode is a fixed GF(2) linear map per erasure pattern.  It is solved at
 // compile time (constexpr Gauss-Jordan over the code's row/diagonal equations)
-// for the built (p, k) configurations, so the kernel is a straight-line XOR
-// network over the surviving cells; other configurations take the same map as
-// a kernel argument.
+// for the full-width codes, so the kernel is a straight-line XOR network over
+// the surviving cells; the other codes form the syndromes and walk the chains.
 #include "rdp_plan.h"
 
 namespace kvec {
@@ -128,6 +127,163 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
 }
 
+// ------------------------------------------------- decode of any pattern
+// Row parity makes P a column like the data: column p-1 of both equations.  So
+// every pattern is at most two lost columns c0 < c1 among the data and P, and
+// Q lost or not, and one kernel per (p, k) serves them all.
+//
+// First the syndromes, as the encode folds its parities: row[r] is the XOR of
+// row r's surviving cells (P's included), diag[d] that of diagonal d's and of
+// Q[d].  Lost shards are read through an empty buffer resource (zeros, no
+// memory traffic), so nothing here depends on the pattern and every diagonal
+// is a compile-time accumulator; the cells of rdp_group(p, k) shards are kept in
+// flight, a shard's requested as an earlier one's are folded.  Then the lost cells, from the syndromes in LDS (each lane its
+// own column, no barrier), at offsets that follow from c0 and c1:
+//   two columns   the chains of the paper (FAST 2004, section 4): from the
+//                 diagonal that meets column c0 in the imaginary row p-1, c1's
+//                 only unknown of it, then c0's cell of that row by row
+//                 parity, then that cell's diagonal, until diagonal p-1; and
+//                 the same from c1.  Together they cover every row once.
+//   one column    its cells are the row syndromes
+//   Q             diag[d] and, of a column rebuilt above, the cell on d
+// Bound by HBM: every cell is read once and folded with two XORs, where the
+// generic map below tests each cell against 2(p-1) outputs with 8 to 16 loads
+// in flight.  A 201 MB stream, 64 KiB stripes, against that map (one box,
+// byte-identical): 8 shards, two lost 43 us (5.8 TB/s) against 79; 10 shards 41
+// against 77; 12 shards and P lost 40 against 104; 5 shards (p = 7) 48 against
+// 59; 3 shards, one lost 54 against 56; a 1 MB stream of 8 shards 11.6 against
+// 43.  Lost shards of 4 GiB and more, past a buffer resource, keep that map.
+struct RdpLoss {
+    int c0, c1;        // lost columns (data shard, or p-1 for P), c0 < c1; -1: none
+    int q;             // Q lost
+    uint32_t absent;   // shards not read, bit by shard index
+};
+
+__device__ __forceinline__ void pin(u32x4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
+
+template <int P, int K>
+__global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) void rdp_decode_chain_kernel(
+        RdpPtrs sh, RdpLoss lost, RdpGeom geo, uint32_t nb) {
+    constexpr int ROWS = P - 1, N = K + 2, G = rdp_group(P, N);
+    __shared__ u32x4 syn[2 * ROWS][kBS];
+    const RdpWave w = rdp_wave(geo, ROWS, blockIdx.x, threadIdx.x);
+    if (w.within >= w.g) return;
+    const uint32_t off = uint32_t(w.base) + w.within, g = uint32_t(w.g);
+    {
+        RdpAcc<P> row[ROWS], diag[ROWS];
+        u32x4 x[G][ROWS];
+        auto load = [&](int s) {
+            // (offsets in the VGPR and soffset 0: the range check of an empty
+            // resource must see the whole offset)
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                    sh.p[s], (short)0, int((lost.absent >> s) & 1 ? 0u : nb), int(kBufWord3));
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r)
+                x[s % G][r] = __builtin_bit_cast(
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + r * g, 0, kAuxLoadNT));
+        };
+#pragma unroll
+        for (int s = 0; s < G; ++s) load(s);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < N; ++s) {
+            const int col = s == K ? P - 1 : s;
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const int d = s == K + 1 ? r : (r + col) % P;
+                if (s <= K) row[r].add(x[s % G][r]);
+                if (d != P - 1) diag[d].add(x[s % G][r]);
+            }
+            if (s + G < N) {
+                // the folds happen here: left free, the compiler put them off
+                // and kept the shards' cells (256 VGPRs and spills)
+                if constexpr (P > 7) {
+#pragma unroll
+                    for (int r = 0; r < ROWS; ++r) {
+                        pin(row[r].a);
+                        pin(diag[r].a);
+                    }
+                }
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                load(s + G);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            syn[r][threadIdx.x] = row[r].get();
+            syn[ROWS + r][threadIdx.x] = diag[r].get();
+        }
+    }
+    auto put = [&](int shard, int r, u32x4 v) { ShardView<true>(sh.p[shard], nb).store(r * g, off, v); };
+    auto shard_of = [&](int col) { return col == P - 1 ? K : col; };
+    auto mod = [](int x) { return x >= P ? x - P : x; };
+    if (lost.c1 >= 0) {
+        // from the diagonal of the imaginary cell (p-1, x): y's cell of it,
+        // then x's of the same row
+        auto chain = [&](int x, int y) {
+            const int sx = shard_of(x), sy = shard_of(y);
+            u32x4 prev = {0, 0, 0, 0};   // x's cell on diagonal d
+            for (int d = mod(x + P - 1); d != P - 1;) {
+                const int r = mod(d + P - y);
+                const u32x4 vy = syn[ROWS + d][threadIdx.x] ^ prev;
+                prev = syn[r][threadIdx.x] ^ vy;
+                put(sy, r, vy);
+                put(sx, r, prev);
+                d = mod(r + x);
+            }
+        };
+        chain(lost.c0, lost.c1);
+        chain(lost.c1, lost.c0);
+        return;
+    }
+    if (lost.c0 >= 0)
+        for (int r = 0; r < ROWS; ++r) put(shard_of(lost.c0), r, syn[r][threadIdx.x]);
+    if (lost.q)
+        for (int d = 0; d < ROWS; ++d) {
+            u32x4 v = syn[ROWS + d][threadIdx.x];
+            const int r = lost.c0 >= 0 ? mod(d + P - lost.c0) : P - 1;
+            if (r != P - 1) v ^= syn[r][threadIdx.x];
+            put(K + 1, d, v);
+        }
+}
+
+typedef void (*ChainFn)(RdpPtrs, RdpLoss, RdpGeom, uint32_t);
+template <int P, int K = 1>
+ChainFn pick_chain(int k) {
+    // k = p - 1 up to p = 7 has the compiled networks
+    if constexpr (K > (P <= 7 ? P - 2 : P - 1)) {
+        return nullptr;
+    } else {
+        if (k == K) return &rdp_decode_chain_kernel<P, K>;
+        return pick_chain<P, K + 1>(k);
+    }
+}
+static ChainFn chain_fn(int p, int k) {
+    switch (p) {
+        case 3: return pick_chain<3>(k);
+        case 5: return pick_chain<5>(k);
+        case 7: return pick_chain<7>(k);
+        case 11: return pick_chain<11>(k);
+        case 13: return pick_chain<13>(k);
+        default: return nullptr;
+    }
+}
+
+// a, or a and b, lost (shard indices, a < b).
+static RdpLoss rdp_loss(int p, int k, int a, int b) {
+    RdpLoss l{-1, -1, 0, 0};
+    for (int e : {a, b}) {
+        if (e < 0) continue;
+        l.absent |= 1u << e;
+        if (e == k + 1) l.q = 1;
+        else (l.c0 < 0 ? l.c0 : l.c1) = e == k ? p - 1 : e;
+    }
+    if (l.c1 < 0) l.absent |= 1u << (k + 1);   // Q serves two lost columns only
+    return l;
+}
+
 // The decode map by input cell, for the generic kernel: each cell the outputs
 // need, with the set of outputs (bit o) that XOR it in.  Built on the host
 // from the plan's per-output masks.
@@ -156,7 +312,8 @@ inline RdpCellMap rdp_cell_map(const RdpPlan& plan) {
     return cm;
 }
 
-// Same map for any (p, k) and any shard size.  Each needed cell is loaded
+// Same map for any (p, k) and any shard size: today shards of 4 GiB and more
+// of the codes without a compiled network.  Each needed cell is loaded
 // once, BATCH at a time so that BATCH are in flight, and folded into every
 // output that uses it (wave-uniform tests of its output set); the 2 ROWS
 // outputs accumulate in registers.  Sized per p, so that small codes keep
@@ -261,8 +418,8 @@ DecFn pick_decode(int e0, int e1) {
 }
 
 // Compile-time XOR networks are built for the full-width codes p = 3, 5, 7,
-// through buffer resources (shards below 4 GiB) or flat addresses (larger);
-// everything else takes the generic kernel.
+// through buffer resources (shards below 4 GiB) or flat addresses (larger); the
+// other codes take the chain kernel below 4 GiB and the generic one above.
 template <bool BUF>
 static DecFn decode_fn_t(int p, int k, int e0, int e1) {
     if (p == 7 && k == 6) return pick_decode<7, 6, BUF>(e0, e1);
@@ -355,8 +512,11 @@ extern "C" int kvec_rdp_decode(void* const* shards, int k, int p, int64_t row_by
     const RdpGeom geo = make_rdp_geom(uint64_t(row_bytes), uint64_t(unit_bytes));
     const dim3 grid(unsigned(rdp_waves(geo))), block(kBS);
     DecFn fn = decode_fn(p, k, a, b, fits_buffer(nb));
+    const ChainFn cfn = fits_buffer(nb) ? chain_fn(p, k) : nullptr;
     if (fn) {
         hipLaunchKernelGGL(fn, grid, block, 0, as_stream(stream), s, geo, nb);
+    } else if (cfn) {
+        hipLaunchKernelGGL(cfn, grid, block, 0, as_stream(stream), s, rdp_loss(p, k, a, b), geo, uint32_t(nb));
     } else {
         RdpPlan plan = make_rdp_plan(p, k, a, b);
         if (!plan.ok)

@@ -146,3 +146,22 @@ def test_rdp_flat_addressing_large_shards(pkg, ora, gpu):
     finally:
         del shards
         torch.cuda.empty_cache()
+
+
+# the chain decode's codes (every k without a compiled network): every pattern
+# of one and two lost shards, short last stripes and rows shorter than a wave
+@pytest.mark.parametrize("p,ks", [(3, [1]), (5, [1, 2, 3]), (7, [1, 3, 5]), (11, [1, 6, 8, 10]), (13, [2, 11, 12])])
+@pytest.mark.parametrize("R,unit", [(16, 0), (1040, 1024), (2064, 0), (5136, 2048)])
+def test_chain_decode_every_pattern(pkg, ora, gpu, p, ks, R, unit):
+    for k in ks:
+        rng = np.random.default_rng(p * 100 + k + R)
+        data = [rng.integers(0, 256, (p - 1) * R, dtype=np.uint8) for _ in range(k)]
+        Pw, Qw = ora.rdp_encode(data, p, unit=unit)
+        want = [torch.from_numpy(np.ascontiguousarray(x).reshape(-1)).to(gpu) for x in (*data, Pw, Qw)]
+        pats = [(a,) for a in range(k + 2)] + [(a, b) for a in range(k + 2) for b in range(a + 1, k + 2)]
+        for pat in pats:
+            sh = [w.clone() for w in want]
+            for e in pat:
+                sh[e].fill_(0x5A)
+            pkg.spec.rdp_decode(sh, p, list(pat), unit_bytes=unit)
+            assert all(torch.equal(a, b) for a, b in zip(sh, want)), (k, pat)
