@@ -90,6 +90,8 @@ SIGNATURES = {
     "kvec_rs8_cauchy": (_i, [_i, _i, _vp]),
     "kvec_rs8_encode": (_i, [_pp, _i, _pp, _i, _i64, _vp]),
     "kvec_rs8_decode": (_i, [_pp, _i, _i, _i64, _vp, _i, _vp]),
+    "kvec_rs8_encode_kv": (_i, [_vp, _vp, _i64, _vp, _i, _i, _i64, _vp]),
+    "kvec_rs8_recover_kv": (_i, [_vp, _vp, _vp, _i64, _i, _i, _i64, _vp, _i, _vp]),
     "kvec_kv_stream_bytes": (_i64, [_kvp]),
     "kvec_kv_gather": (_i, [_kvp, _vp, _vp]),
     "kvec_kv_gather_split": (_i, [_kvp, _vp, _vp, _vp]),

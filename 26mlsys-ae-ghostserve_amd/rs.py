@@ -117,6 +117,12 @@ def shard_size_and_pad(total_symbols: int, num_data_shards: int):
 SCHEMES = ("ghostserve", "spec")
 
 
+def _rows_in_range(scheme: str, k: int, m: int) -> bool:
+    """Whether the one-pass entry points may be asked (the GF(2^8) one refuses
+    codes past its limits, which the general path then reports)."""
+    return scheme == "ghostserve" or (1 <= k <= 32 and 1 <= m <= 4 and k * m <= 64)
+
+
 def forward_encode_kv(keys: torch.Tensor, values: torch.Tensor, num_data_shards: int,
                       num_parity_shards: int, scheme: str = "ghostserve"):
     """benchmark/rs/main.py:63-137: returns (shards [(k+m), S] uint16, meta).
@@ -145,10 +151,12 @@ def forward_encode_kv(keys: torch.Tensor, values: torch.Tensor, num_data_shards:
     keys = keys.contiguous()
     values = values.contiguous()
     # one pass over K and V for the rows and the parity, when the layout allows it
-    if not (scheme == "ghostserve" and N_k == N_v and
-            _lib.call_if_built("kvec_rs16_encode_kv", keys.data_ptr(), values.data_ptr(), 2 * N_k,
+    name, S = (("kvec_rs16_encode_kv", shard_sz) if scheme == "ghostserve"
+               else ("kvec_rs8_encode_kv", 2 * shard_sz))
+    if not (N_k == N_v and _rows_in_range(scheme, num_data_shards, num_parity_shards) and
+            _lib.call_if_built(name, keys.data_ptr(), values.data_ptr(), 2 * N_k,
                                shards.data_ptr(), int(num_data_shards), int(num_parity_shards),
-                               int(shard_sz), _stream(shards))):
+                               int(S), _stream(shards))):
         # K || V and the zero padding go straight into the shard tensor's data
         # rows (the reference packs into a separate data_padded and the encode
         # copies it over); the encode then reads the rows in place and writes
@@ -200,24 +208,34 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
     if len(missing_data) > len(avail_par):
         raise RuntimeError("Not enough parity shards to reconstruct the missing data shards.")
 
-    if meta.get("scheme", "ghostserve") == "spec":
-        if len(set(missing_shards)) > num_parity:
-            raise RuntimeError("Not enough parity shards to reconstruct the missing shards.")
-        if missing_shards:
-            rows = shards.view(torch.uint8).view(num_data + num_parity, -1)
-            spec.rs8_decode([rows[i] for i in range(num_data + num_parity)], num_data,
-                            [int(i) for i in missing_shards])
-        missing_data = []
+    is_spec = meta.get("scheme", "ghostserve") == "spec"
+    if is_spec and len(set(missing_shards)) > num_parity:
+        raise RuntimeError("Not enough parity shards to reconstruct the missing shards.")
     dtype = meta.get("dtype", torch.float16)
     N_k, N_v = meta["N_k"], meta["N_v"]
     B, H, T, D = meta["B"], meta["H"], meta["T"], meta["D"]
     K = torch.empty(N_k, dtype=dtype, device=device)
     V = torch.empty(N_v, dtype=dtype, device=device)
+    one_pass = (N_k == N_v and shards.is_cuda and shards.is_contiguous() and
+                K.element_size() == 2 and shards.element_size() == 2)
+    if is_spec:
+        if missing_shards:
+            lost = np.ascontiguousarray([int(i) for i in missing_shards], dtype=np.int32)
+            if (one_pass and lost.max() < num_data + num_parity
+                    and _rows_in_range("spec", num_data, num_parity)
+                    and _lib.call_if_built("kvec_rs8_recover_kv", shards.data_ptr(), K.data_ptr(),
+                                           V.data_ptr(), 2 * int(N_k), int(num_data),
+                                           int(num_parity), 2 * int(shard_sz), lost.ctypes.data,
+                                           int(lost.size), _stream(shards))):
+                return K.view(B, H, T, D), V.view(B, H, T, D)
+            rows = shards.view(torch.uint8).view(num_data + num_parity, -1)
+            spec.rs8_decode([rows[i] for i in range(num_data + num_parity)], num_data,
+                            [int(i) for i in missing_shards])
+        missing_data = []
     # the rebuild and the split in one pass when the first parity rows serve
     # and the layout allows it
-    if (missing_data and N_k == N_v and avail_par[:len(missing_data)] == list(range(len(missing_data)))
-            and shards.is_cuda and shards.is_contiguous()
-            and K.element_size() == 2 and shards.element_size() == 2):
+    if (one_pass and missing_data and
+            avail_par[:len(missing_data)] == list(range(len(missing_data)))):
         lost = np.asarray(missing_data, dtype=np.int32)
         if _lib.call_if_built("kvec_rs16_recover_kv", shards.data_ptr(), K.data_ptr(), V.data_ptr(),
                               2 * int(N_k), int(num_data), int(num_parity), int(shard_sz),

@@ -97,6 +97,20 @@ int kvec_rs8_encode(const void* const* data, int k, void* const* parity, int m,
 int kvec_rs8_decode(void* const* shards, int k, int m, int64_t shard_bytes,
                     const int32_t* erased, int n_erased, void* stream);
 
+/* The spec scheme of forward_encode_kv / backwards_decode_kv (benchmark/rs/main.py
+ * :63-206) in one pass each, on a packed [(k+m)][row_bytes] tensor.  Encode: the
+ * data rows are K || V || zeros (kv_half_bytes raw bytes each), the parity rows
+ * those of kvec_rs8_encode.  Recover: the erased rows (host int32 array, data or
+ * parity) rebuilt in place as by kvec_rs8_decode and the rows' first
+ * 2*kv_half_bytes bytes written to K and V.  KVEC_EUNSUPPORTED, with nothing
+ * enqueued, outside: 1 to 4 parity (erased) rows, K, V, shards and kv_half_bytes
+ * multiples of 16, K and V below 1 GiB, shards below 2 GiB. */
+int kvec_rs8_encode_kv(const void* key_input, const void* value_input, int64_t kv_half_bytes, void* shards,
+                       int data_shards, int parity_shards, int64_t row_bytes, void* stream);
+int kvec_rs8_recover_kv(void* shards, void* key_output, void* value_output, int64_t kv_half_bytes,
+                        int data_shards, int parity_shards, int64_t row_bytes, const int32_t* erased, int n_erased,
+                        void* stream);
+
 /* ============================ paged KV gather ============================ */
 /* The delta gather of the serving plugin, K = pool[slots, 0], V = pool[slots, 1]
  * (bench_ghostserve_rdp.py:440-458), over a paged pool.  Pool layout:

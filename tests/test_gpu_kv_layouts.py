@@ -105,3 +105,73 @@ def _rs16_round(pkg, ora, gpu, k, m, B, H, T, D):
         assert torch.equal(sh.view(torch.int16), full.view(torch.int16)), er
         assert torch.equal(k2.view(torch.int16), K.view(torch.int16)), er
         assert torch.equal(v2.view(torch.int16), V.view(torch.int16)), er
+
+
+# GF(2^8) codes behind the same wrappers: one to four outputs in one pass (five
+# parities: the pack and the shard kernels), odd and even k, rows of one chunk,
+# a tile, tiles and a remainder; every parity row and mixes of lost rows
+@pytest.mark.parametrize("k,m", [(1, 1), (4, 1), (5, 3), (6, 2), (8, 4), (10, 4), (16, 2), (9, 3), (6, 5)])
+@pytest.mark.parametrize("B,H,T,D", [(1, 1, 9, 8), (1, 2, 33, 128), (2, 3, 101, 80), (1, 8, 512, 128), (3, 4, 521, 128)])
+def test_rs8_kv(pkg, ora, gpu, k, m, B, H, T, D):
+    K, V = _kv(B, H, T, D, "head", gpu, seed=k)
+    sh, meta = pkg.rs.forward_encode_kv(K, V, k, m, scheme="spec")
+    S = meta["shard_sz"]
+    data = np.zeros(k * S, np.uint16)
+    flat = np.concatenate([x.view(torch.int16).cpu().numpy().reshape(-1).view(np.uint16) for x in (K, V)])
+    data[:flat.size] = flat
+    rows = data.view(np.uint8).reshape(k, 2 * S)
+    par = ora.rs8_encode([r.copy() for r in rows], m)
+    want = np.concatenate([rows.reshape(-1)] + [np.asarray(p).reshape(-1) for p in par])
+    assert np.array_equal(sh.cpu().numpy().view(np.uint8).reshape(-1), want)
+    full = sh.clone()
+    lost = [[e] for e in range(k + m)] + [list(range(min(m, k))), list(range(k + m - m, k + m))]
+    lost += [[0, k + m - 1], [k - 1, k]] if m > 1 else []
+    for er in lost:
+        sh.copy_(full)
+        for e in er:
+            sh.view(torch.int16)[e] = 0x5A5A
+        k2, v2 = pkg.rs.backwards_decode_kv(sh, meta, er)
+        assert torch.equal(sh.view(torch.int16), full.view(torch.int16)), er
+        assert torch.equal(k2.view(torch.int16), K.view(torch.int16)), er
+        assert torch.equal(v2.view(torch.int16), V.view(torch.int16)), er
+
+
+# separate shards of the shapes without a straight-line kernel: groups of four
+# outputs and a remainder, odd and even input counts, shards of one chunk, a
+# tile, a tile and a chunk
+@pytest.mark.parametrize("k,m", [(8, 3), (8, 4), (6, 3), (12, 4), (16, 2), (8, 8), (9, 7), (32, 2), (1, 1), (3, 2)])
+@pytest.mark.parametrize("S", [16, 8192, 8192 * 2 + 16, 70000])
+def test_rs8_loop_shapes(pkg, ora, gpu, k, m, S):
+    rng = np.random.default_rng(k * 10 + m)
+    data = [rng.integers(0, 256, S, dtype=np.uint8) for _ in range(k)]
+    par = [np.asarray(p).reshape(-1) for p in ora.rs8_encode(data, m)]
+    want = [torch.from_numpy(x.copy()).to(gpu) for x in data + par]
+    sh = [w.clone() for w in want]
+    for p in sh[k:]:
+        p.zero_()
+    pkg.spec.rs8_encode(sh[:k], sh[k:])
+    assert all(torch.equal(a, b) for a, b in zip(sh, want))
+    for er in ([0], list(range(min(k, m))), list(range(k + m - m, k + m)), sorted({0, k + m - 1} if m > 1 else {k})):
+        for e in er:
+            sh[e].fill_(0x5A)
+        pkg.spec.rs8_decode(sh, k, er)
+        assert all(torch.equal(a, b) for a, b in zip(sh, want)), er
+
+
+# both sides of the size from which two outputs of four to six inputs are coded
+# straight-line
+@pytest.mark.parametrize("k", [4, 5, 6])
+@pytest.mark.parametrize("S", [(60 << 20) - 16, 60 << 20, (60 << 20) + 1040])
+def test_rs8_straight_line_sizes(pkg, ora, gpu, k, S):
+    g = torch.Generator(device=gpu).manual_seed(k)
+    data = [torch.randint(-2**62, 2**62, (S // 8,), generator=g, device=gpu).view(torch.uint8) for _ in range(k)]
+    par = [torch.empty_like(d) for d in data[:2]]
+    pkg.spec.rs8_encode(data, par)
+    at = torch.cat([torch.arange(0, 16 * 1024), torch.arange(S - 16 * 1024, S)]).to(gpu)
+    want = ora.rs8_encode([d[at].cpu().numpy() for d in data], 2)
+    assert all(np.array_equal(p[at].cpu().numpy(), np.asarray(w).reshape(-1)) for p, w in zip(par, want))
+    full = [d.clone() for d in data[:2]]
+    data[0].zero_()
+    data[1].zero_()
+    pkg.spec.rs8_decode(data + par, k, [0, 1])
+    assert torch.equal(data[0], full[0]) and torch.equal(data[1], full[1])
