@@ -111,6 +111,8 @@ SIGNATURES = {
     "kvec_gs_rdp_recover": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _i, _i, _vp]),
     "kvec_gs_rdp_backup_kv": (_i, [_kbp, _vp, _i, _i, _i, _vp]),
     "kvec_gs_rdp_recover_kv": (_i, [_vp, _kbp, _i, _i, _i, _i, _i, _vp]),
+    "kvec_kv_pack_bhtd": (_i, [_kbp, _vp, _i64, _vp]),
+    "kvec_kv_unpack_bhtd": (_i, [_vp, _i64, _kbp, _vp]),
     "kvec_gs_pack_row": (_i, [_vp, _vp, _vp, _i64, _i, _i64, _vp]),
     "kvec_gs_rdp_parity": (_i, [_vp, _i, _i, _i, _vp]),
     "kvec_hook_step": (_i, [_kvp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _pp]),

@@ -32,24 +32,28 @@ __device__ __forceinline__ u32x4 drop_word(u32x4 v, int64_t k) {
     return v;
 }
 
-// Per data row r < 8: the diagonal its star word lies on, (star_r + r) mod S
+// Per data row r < 16: the diagonal its star word lies on, (star_r + r) mod S
 // with star_r = (star_base + r) % S, or -1 when the row skips nothing (C
 // remainder: a negative star_base gives a negative star_r).  The same for
 // every tile, so the host computes it once; the batched path runs only on
 // row tensors below 2 GiB, so it fits 32 bits.
+constexpr int kGsMaxRows = 16;   // rows of the one-tile kernels
 struct GsStar {
-    int32_t d[8];
+    int32_t d[kGsMaxRows];
 };
 
 inline GsStar make_gs_star(int star_base, int64_t S) {
     GsStar star{};
-    for (int r = 0; r < 8; ++r) {
+    for (int r = 0; r < kGsMaxRows; ++r) {
         const int64_t sr = (int64_t(star_base) + r) % S;
         star.d[r] = sr < 0 ? -1 : int32_t((sr + r) % S);
     }
     return star;
 }
 
+// P and Q of 9 .. kGsMaxRows rows of S >= 64 words in a tensor whose bytes fit
+// the kernels' resources, gs_kv.hip.
+int gs_rdp_parity_wide(uint16_t* sh, int nd, int64_t S, int star_base, hipStream_t st, const char* what);
 // The data row a recovery rebuilds, gs_xor_rdp.hip.
 int gs_recover_row(int nd, int S, int star_base, int missing_a, int missing_b, const char* fn, int* row);
 

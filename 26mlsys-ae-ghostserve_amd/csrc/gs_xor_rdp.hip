@@ -798,6 +798,8 @@ static int gs_rdp_parity(uint16_t* sh, int nd, int64_t S, int star_base, hipStre
     const uint64_t lim = (uint64_t(1) << 31) - 16;
     const bool small = rows_bytes <= lim && (!fused || uint64_t(fused->kb) <= lim);
     const uint64_t rb = small ? rows_bytes : 0;
+    if (!fused && small && nd > 8 && nd <= kGsMaxRows && S >= 64)
+        return gs_rdp_parity_wide(sh, nd, S, star_base, st, what);
     const GsStar star = make_gs_star(star_base, S);
     if (fused)
         hipLaunchKernelGGL(gs_parity_fn<true>(nd), grid, dim3(kTB), 0, st, sh, nd, S, star_base, *fused, rb,
@@ -1018,7 +1020,9 @@ extern "C" int kvec_gs_rdp_backup(const void* K_TN, const void* V_TN, void* shar
         const uintptr_t R0 = uintptr_t(shards), Rend = R0 + (cap + 2 * uint64_t(S)) * 2;
         const uintptr_t Kp = uintptr_t(K_TN), Vp = uintptr_t(V_TN);
         const bool apart = (Kp + tn * 2 <= R0 || Kp >= Rend) && (Vp + tn * 2 <= R0 || Vp >= Rend);
-        if (apart && ((Kp ^ R0) & 15) == 0 && ((Vp ^ (R0 + tn * 2)) & 15) == 0) {
+        // Nine to sixteen rows, which that kernel takes one at a time, are copied
+        // and then coded with every row in flight.
+        if (apart && (nd <= 8 || nd > kGsMaxRows || S < 64) && ((Kp ^ R0) & 15) == 0 && ((Vp ^ (R0 + tn * 2)) & 15) == 0) {
             const uint64_t kv = 4 * tn, rows = 2 * cap;
             const GsSource g{(const uint8_t*)K_TN, (const uint8_t*)V_TN, int64_t(2 * tn),
                              int64_t(kv < rows ? kv : rows), int64_t(Rend - R0)};

@@ -94,6 +94,11 @@ def _check_scheme(scheme: str):
         raise ValueError(f"scheme must be one of {SCHEMES}, not {scheme!r}")
 
 
+def _token_major(keys, values):
+    """[T, B*H*D] copies of K and V indexed [B, H, T, D]."""
+    return tuple(x.permute(2, 0, 1, 3).contiguous().view(x.shape[2], -1) for x in (keys, values))
+
+
 def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
                          num_data_shards: int, star_base: int = 0, scheme: str = "ghostserve"):
     """benchmark/rdp/main.py:44-92: token-major pack + P/Q in one call.
@@ -125,24 +130,26 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
     t0.record()
     # one pass over K and V where they lie, when their layout allows it; else
     # token-major copies, then the pack and the code
-    kv = _lib.kv_bhtd(keys_bhtd, values_bhtd) if scheme == "ghostserve" else None
-    if kv is None or not _lib.call_if_built("kvec_gs_rdp_backup_kv", kv, shards.data_ptr(), nd,
-                                            int(shard_size), int(star_base), _stream(shards)):
-        K_TN = keys_bhtd.permute(2, 0, 1, 3).contiguous().view(T, n)
-        V_TN = values_bhtd.permute(2, 0, 1, 3).contiguous().view(T, n)
+    kv = _lib.kv_bhtd(keys_bhtd, values_bhtd)
+    if scheme == "spec":
+        if kv is None or not _lib.call_if_built("kvec_kv_pack_bhtd", kv, shards.data_ptr(),
+                                                2 * nd * int(shard_size), _stream(shards)):
+            K_TN, V_TN = _token_major(keys_bhtd, values_bhtd)
+            shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
+            t0.record()
+            _lib.call("kvec_rs16_pack", K_TN.data_ptr(), V_TN.data_ptr(), shards.data_ptr(),
+                      T * n, T * n, _stream(shards))
+        rows = _rows_u8(shards)
+        spec.rdp_encode(rows[:nd], rows[nd], rows[nd + 1], p, unit_bytes=spec.RDP_UNIT)
+    elif kv is None or not _lib.call_if_built("kvec_gs_rdp_backup_kv", kv, shards.data_ptr(), nd,
+                                              int(shard_size), int(star_base), _stream(shards)):
+        K_TN, V_TN = _token_major(keys_bhtd, values_bhtd)
         # the reference zero-fills everything; only the padding words are read
         # before being written
         shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
         t0.record()
-        if scheme == "spec":
-            # K_TN || V_TN into the data rows, then textbook RDP over the rows
-            _lib.call("kvec_rs16_pack", K_TN.data_ptr(), V_TN.data_ptr(), shards.data_ptr(),
-                      T * n, T * n, _stream(shards))
-            rows = _rows_u8(shards)
-            spec.rdp_encode(rows[:nd], rows[nd], rows[nd + 1], p, unit_bytes=spec.RDP_UNIT)
-        else:
-            rdp_kernel.fused_backup_full_kv(K_TN, V_TN, shards, nd, int(shard_size), int(T),
-                                            int(n), int(star_base))
+        rdp_kernel.fused_backup_full_kv(K_TN, V_TN, shards, nd, int(shard_size), int(T), int(n),
+                                        int(star_base))
     t1.record()
     torch.cuda.synchronize()
     backup_ms = t0.elapsed_time(t1)
@@ -184,15 +191,20 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
     t0.record()
     # the rows written straight to K and V when the layout allows it; else
     # through a token-major copy
-    direct = (pkg.get("scheme", "ghostserve") != "spec" and
-              _lib.call_if_built("kvec_gs_rdp_recover_kv", shards.data_ptr(),
-                                 _lib.kv_bhtd(keys, values), int(nd), int(shard_size),
-                                 int(star_base), int(missing_a), int(missing_b), _stream(shards)))
+    kv = _lib.kv_bhtd(keys, values)
+    is_spec = pkg.get("scheme", "ghostserve") == "spec"
+    if is_spec:
+        lost = [int(e) for e in (missing_a, missing_b) if 0 <= int(e) < nd + 2]
+        spec.rdp_decode(_rows_u8(shards), int(pkg["p"]), lost, unit_bytes=spec.RDP_UNIT)
+        direct = _lib.call_if_built("kvec_kv_unpack_bhtd", shards.data_ptr(),
+                                    2 * int(nd) * int(shard_size), kv, _stream(shards))
+    else:
+        direct = _lib.call_if_built("kvec_gs_rdp_recover_kv", shards.data_ptr(), kv, int(nd),
+                                    int(shard_size), int(star_base), int(missing_a),
+                                    int(missing_b), _stream(shards))
     if not direct:
         packed_TN = torch.empty(2 * T * n, dtype=dtype, device=shards.device)
-        if pkg.get("scheme", "ghostserve") == "spec":
-            lost = [int(e) for e in (missing_a, missing_b) if 0 <= int(e) < nd + 2]
-            spec.rdp_decode(_rows_u8(shards), int(pkg["p"]), lost, unit_bytes=spec.RDP_UNIT)
+        if is_spec:
             _lib.call("kvec_rs16_split", shards.data_ptr(), packed_TN.data_ptr(),
                       packed_TN[T * n:].data_ptr(), T * n, T * n, _stream(shards))
         else:

@@ -282,12 +282,18 @@ typedef struct kvec_kv_bhtd {
  * zeros read from K and V where they lie, then P and Q as kvec_gs_rdp_backup.
  * Every byte of shards is written.  KVEC_EUNSUPPORTED, with nothing enqueued,
  * for layouts it does not take: head_bytes, strides or pointers not multiples
- * of 16, nd > 8, S < 64, K or V over 1 GiB, shards of 2 GiB. */
+ * of 16, nd > 12 (recovery: 16), S < 64, K or V over 1 GiB, shards of 2 GiB. */
 int kvec_gs_rdp_backup_kv(const kvec_kv_bhtd* kv, void* shards, int nd, int S, int star_base, void* stream);
 /* fused_recovery_full_kv, benchmark/rdp/main.py:95-126: the row rebuilt as by
  * kvec_gs_rdp_recover, and the stream written to kv->k and kv->v.  Same limits. */
 int kvec_gs_rdp_recover_kv(void* shards, const kvec_kv_bhtd* kv, int nd, int S, int star_base, int missing_a,
                            int missing_b, void* stream);
+/* The same token-major stream to rows_bytes of rows (zeros past V), and back
+ * (the stream's bytes of rows to K and V): the layout step of the spec scheme
+ * (benchmark/rdp/main.py:60-66, :120-124).  KVEC_EUNSUPPORTED as above, and for
+ * rows_bytes not a multiple of 16 or below the stream's. */
+int kvec_kv_pack_bhtd(const kvec_kv_bhtd* kv, void* rows, int64_t rows_bytes, void* stream);
+int kvec_kv_unpack_bhtd(const void* rows, int64_t rows_bytes, const kvec_kv_bhtd* kv, void* stream);
 /* pack_row_from_block_launcher, bench_ghostserve_rdp.py:152-175:
  * rows[row*S ..] = k_blk words then v_blk words (S >= 2*words). */
 int kvec_gs_pack_row(const void* k_blk, const void* v_blk, void* rows, int64_t words, int row,

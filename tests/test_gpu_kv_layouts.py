@@ -41,7 +41,10 @@ def _tn(x):
 @pytest.mark.parametrize("B,H,T,D,nd", [
     (1, 8, 512, 128, 8), (2, 1, 33, 128, 6), (1, 2, 5, 64, 3), (3, 2, 17, 80, 7), (1, 1, 64, 128, 8),
     (2, 4, 101, 128, 5), (1, 1, 1024, 8, 4), (1, 3, 7, 16, 2), (4, 8, 263, 128, 1), (4, 8, 521, 128, 2),
-    (8, 8, 800, 128, 6), (1, 2, 4096, 64, 1)])
+    (8, 8, 800, 128, 6), (1, 2, 4096, 64, 1),
+    # nine rows and more: two edge chunks; past twelve the backup copies first
+    (1, 8, 512, 128, 9), (2, 3, 101, 80, 10), (1, 2, 37, 128, 12), (1, 2, 37, 128, 13), (2, 4, 203, 64, 16),
+    (8, 8, 2053, 128, 10), (1, 1, 9, 64, 17)])
 @pytest.mark.parametrize("order", ["head", "token", "wide", "odd"])
 def test_gs_rdp_kv_layouts(pkg, ora, gpu, B, H, T, D, nd, order):
     K, V = _kv(B, H, T, D, order, gpu)
@@ -175,3 +178,43 @@ def test_rs8_straight_line_sizes(pkg, ora, gpu, k, S):
     data[1].zero_()
     pkg.spec.rs8_decode(data + par, k, [0, 1])
     assert torch.equal(data[0], full[0]) and torch.equal(data[1], full[1])
+
+
+# P and Q of rows in place, nine to sixteen of them: every word alignment of the
+# tensor, rows of exactly a tile, odd lengths, star words in the wrapped part
+@pytest.mark.parametrize("nd", range(9, 17))
+@pytest.mark.parametrize("soff,S,sb", [(0, 1024, 0), (3, 4096, -1), (5, 6149, 4090), (0, 64, 3), (7, 20481, 2),
+                                       (1, 65, 60), (6, 530003, 0)])
+def test_gs_parity_wide(pkg, ora, gpu, nd, soff, S, sb):
+    rng = np.random.default_rng(nd + S)
+    rows = rng.integers(0, 65536, (nd + 2, S), dtype=np.uint16)
+    want = rows.copy()
+    ora.gs_parity(want, nd, S, sb)
+    buf = torch.full(((nd + 2) * S + 32,), 0x3C3C, dtype=torch.int16, device=gpu)
+    buf[soff:soff + rows.size] = torch.from_numpy(rows.reshape(-1).view(np.int16)).to(gpu)
+    pkg.rdp_kv_ops.compute_rdp_parity(buf.view(torch.uint16)[soff:soff + rows.size].view(nd + 2, S), nd, S, sb)
+    got = buf.cpu().numpy().view(np.uint16)
+    assert np.array_equal(got[soff:soff + rows.size], want.reshape(-1))
+    assert (np.concatenate([got[:soff], got[soff + rows.size:]]) == 0x3C3C).all()
+
+
+# the spec scheme's layout step from and to strided K and V
+@pytest.mark.parametrize("B,H,T,D,nd", [(1, 8, 512, 128, 8), (3, 2, 17, 80, 5), (2, 4, 1301, 128, 6), (1, 1, 5, 8, 2)])
+@pytest.mark.parametrize("order", ["head", "token", "wide", "odd"])
+def test_rdp_spec_kv_layouts(pkg, ora, gpu, B, H, T, D, nd, order):
+    K, V = _kv(B, H, T, D, order, gpu)
+    pk = pkg.rdp.fused_backup_full_kv(K, V, nd, scheme="spec")
+    S, n = pk["shard_size"], 2 * B * H * T * D
+    flat = np.zeros(nd * S, np.uint16)
+    flat[:n] = np.concatenate([_tn(K).reshape(-1), _tn(V).reshape(-1)])
+    rows = flat.view(np.uint8).reshape(nd, 2 * S)
+    Pw, Qw = ora.rdp_encode([r.copy() for r in rows], pk["p"], unit=pkg.spec.RDP_UNIT)
+    got = pk["shards_KV"].cpu().numpy().view(np.uint8)
+    assert np.array_equal(got[:nd], rows)
+    assert np.array_equal(got[nd], Pw.reshape(-1)) and np.array_equal(got[nd + 1], Qw.reshape(-1))
+    pk["shards_KV"].view(torch.int16)[nd - 1] = 0x5A5A
+    pk["shards_KV"].view(torch.int16)[0] = 0x5A5A
+    k2, v2, _ = pkg.rdp.fused_recovery_full_kv(pk, 0, nd - 1)
+    assert np.array_equal(pk["shards_KV"].cpu().numpy().view(np.uint8), got)
+    assert torch.equal(k2.view(torch.int16), K.view(torch.int16).contiguous())
+    assert torch.equal(v2.view(torch.int16), V.view(torch.int16).contiguous())
