@@ -226,44 +226,46 @@ __global__ __launch_bounds__(kPackBS) void kv_rows_kernel(KvStream s, uint8_t* r
 }
 
 // ---------------------------------------------------------------- host side
-// Threads per tile: 512 (8 KiB tiles), or 128 where those would leave most of
-// the 256 compute units idle.
-constexpr int kKvBS = 512, kKvSmallBS = 128;
-constexpr uint64_t kKvSmallTiles = 512;
+// Threads per tile: 512 (8 KiB tiles) up to eight rows and 256 past them, whose
+// registers leave room for 12 waves a CU (16 rows of 8.2 MB, P and Q: 28.9 us
+// against 30.9 with 128 threads and 38.8 with 512; ten rows of K and V, 134 MB:
+// 65.5 against 68.3 and 74.7); 128 where those tiles would leave compute units
+// idle (16 rows of 0.4 MB: 6.7 against 7.3 us with 256).
+constexpr int wide_bs(int nd) { return nd > 8 ? 256 : 512; }
+constexpr int kKvSmallBS = 128;
+static bool small_tiles(int nd, uint64_t Sb) { return Sb < (nd > 8 ? 1u << 20 : 4u << 20); }
 
 constexpr int kKvMaxRows = 12;   // backup from K and V (SGPRs spill from 15 rows on)
 
 typedef void (*BackupKvFn)(KvStream, uint8_t*, uint32_t, GsStar);
 typedef void (*RecoverKvFn)(uint8_t*, uint32_t, uint32_t, int, KvStream);
 
-template <int BS, PqSource SRC, int ND = SRC == kRows ? 9 : 1>
+template <bool SMALL, PqSource SRC, int ND = SRC == kRows ? 9 : 1>
 static BackupKvFn backup_kv_fn(int nd) {
     if constexpr (ND > (SRC == kRows ? kGsMaxRows : kKvMaxRows)) {
         return nullptr;
     } else {
-        if (nd == ND) return &gs_backup_kv_kernel<ND, BS, SRC>;
-        return backup_kv_fn<BS, SRC, ND + 1>(nd);
+        if (nd == ND) return &gs_backup_kv_kernel<ND, SMALL ? kKvSmallBS : wide_bs(ND), SRC>;
+        return backup_kv_fn<SMALL, SRC, ND + 1>(nd);
     }
 }
-template <int BS, bool FLAT, int ND = 1>
+template <bool SMALL, bool FLAT, int ND = 1>
 static RecoverKvFn recover_kv_fn(int nd) {
     if constexpr (ND > kGsMaxRows) {
         return nullptr;
     } else {
-        if (nd == ND) return &gs_recover_kv_kernel<ND, BS, FLAT>;
-        return recover_kv_fn<BS, FLAT, ND + 1>(nd);
+        if (nd == ND) return &gs_recover_kv_kernel<ND, SMALL ? kKvSmallBS : wide_bs(ND), FLAT>;
+        return recover_kv_fn<SMALL, FLAT, ND + 1>(nd);
     }
 }
-
-static bool small_tiles(uint64_t Sb) { return (Sb + 16 * kKvBS - 1) / (16 * kKvBS) < kKvSmallTiles; }
 
 // P and Q (and, from K and V, the data rows) of rows of Sb bytes.
 template <PqSource SRC>
 static int launch_pq(const KvStream& s, uint8_t* sh, int nd, int64_t S, int star_base, hipStream_t st, const char* fn) {
     const uint64_t Sb = uint64_t(S) * 2;
-    const bool small = small_tiles(Sb);
-    const BackupKvFn f = small ? backup_kv_fn<kKvSmallBS, SRC>(nd) : backup_kv_fn<kKvBS, SRC>(nd);
-    const int bs = small ? kKvSmallBS : kKvBS;
+    const bool small = small_tiles(nd, Sb);
+    const BackupKvFn f = small ? backup_kv_fn<true, SRC>(nd) : backup_kv_fn<false, SRC>(nd);
+    const int bs = small ? kKvSmallBS : wide_bs(nd);
     hipLaunchKernelGGL(f, dim3(blocks_for(int64_t(Sb), 16 * bs)), dim3(bs), 0, st, s, sh, uint32_t(Sb),
                        make_gs_star(star_base, S));
     return check_launch(fn);
@@ -321,10 +323,10 @@ extern "C" int kvec_gs_rdp_recover_kv(void* shards, const kvec_kv_bhtd* kv, int 
     if (int rc = gs_recover_row(nd, S, star_base, missing_a, missing_b, fn, &t)) return rc;
     const Span w[3] = {{shards, uint64_t(nd + 2) * Sb, "shards", -1}, {kv->k, s.ext, "k", -1}, {kv->v, s.ext, "v", -1}};
     if (int rc = check_no_alias(w, 3, nullptr, 0, fn)) return rc;
-    const bool small = small_tiles(Sb);
-    const RecoverKvFn f = small ? (flat ? recover_kv_fn<kKvSmallBS, true>(nd) : recover_kv_fn<kKvSmallBS, false>(nd))
-                                : (flat ? recover_kv_fn<kKvBS, true>(nd) : recover_kv_fn<kKvBS, false>(nd));
-    const int bs = small ? kKvSmallBS : kKvBS;
+    const bool small = small_tiles(nd, Sb);
+    const RecoverKvFn f = small ? (flat ? recover_kv_fn<true, true>(nd) : recover_kv_fn<true, false>(nd))
+                                : (flat ? recover_kv_fn<false, true>(nd) : recover_kv_fn<false, false>(nd));
+    const int bs = small ? kKvSmallBS : wide_bs(nd);
     hipLaunchKernelGGL(f, dim3(blocks_for(int64_t(Sb), 16 * bs)), dim3(bs), 0, as_stream(stream), (uint8_t*)shards,
                        uint32_t(Sb), uint32_t(uint64_t(nd + 1) * Sb), t, s);
     return check_launch(fn);
