@@ -145,7 +145,7 @@ def backwards_decode_kv(pkg, missing_shards):
     # call (one pass over the rows when a data row is lost).  The reference
     # zeroes the missing shard first; that row is rewritten in full and never
     # read, so the zeroing is left out.
-    es = torch.empty((), dtype=dtype).element_size()
+    es = dtype.itemsize
     de_bytes_needed = 2 * es * T * n
     if num_data_shards * shard_size < de_bytes_needed:
         raise RuntimeError("Not enough bytes in reconstructed data region.")
