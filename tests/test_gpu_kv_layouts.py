@@ -218,3 +218,39 @@ def test_rdp_spec_kv_layouts(pkg, ora, gpu, B, H, T, D, nd, order):
     assert np.array_equal(pk["shards_KV"].cpu().numpy().view(np.uint8), got)
     assert torch.equal(k2.view(torch.int16), K.view(torch.int16).contiguous())
     assert torch.equal(v2.view(torch.int16), V.view(torch.int16).contiguous())
+
+
+@pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
+def test_rs_kv_graph_replay(pkg, gpu, scheme):
+    """The one-pass encode and decode captured in one graph: every replay on
+    fresh K and V, with eager calls between replays, gives the eager bytes."""
+    k, m, lost = 6, 2, [1, 4]
+    K, V = _kv(2, 4, 203, 128, "head", gpu)
+    full, meta = pkg.rs.forward_encode_kv(K, V, k, m, scheme=scheme)   # tables and library loaded
+
+    def step():
+        sh, _ = pkg.rs.forward_encode_kv(K, V, k, m, scheme=scheme)
+        before = sh.clone()
+        for e in lost:
+            sh.view(torch.int16)[e].fill_(0x5A5A)
+        return before, sh, *pkg.rs.backwards_decode_kv(sh, meta, lost)
+
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        step()
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        before, sh, k2, v2 = step()
+    for i in range(4):
+        x, y = _kv(2, 4, 203, 128, "head", gpu, seed=100 + i)
+        K.copy_(x)
+        V.copy_(y)
+        want, _ = pkg.rs.forward_encode_kv(x, y, k, m, scheme=scheme)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(before.view(torch.int16), want.view(torch.int16)), i
+        assert torch.equal(sh.view(torch.int16), want.view(torch.int16)), i
+        assert torch.equal(k2.view(torch.int16), x.view(torch.int16)), i
+        assert torch.equal(v2.view(torch.int16), y.view(torch.int16)), i
