@@ -150,6 +150,7 @@ def forward_encode_kv(keys: torch.Tensor, values: torch.Tensor, num_data_shards:
     shards = torch.empty((total_shards, shard_sz), dtype=torch.uint16, device=device)
     keys = keys.contiguous()
     values = values.contiguous()
+    _lib.require_cuda(keys, values, shards, what="forward_encode_kv tensor")
     # one pass over K and V for the rows and the parity, when the layout allows it
     name, S = (("kvec_rs16_encode_kv", shard_sz) if scheme == "ghostserve"
                else ("kvec_rs8_encode_kv", 2 * shard_sz))

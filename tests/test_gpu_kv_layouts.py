@@ -254,3 +254,17 @@ def test_rs_kv_graph_replay(pkg, gpu, scheme):
         assert torch.equal(sh.view(torch.int16), want.view(torch.int16)), i
         assert torch.equal(k2.view(torch.int16), x.view(torch.int16)), i
         assert torch.equal(v2.view(torch.int16), y.view(torch.int16)), i
+
+
+@pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
+def test_rs_encode_refuses_host_values(pkg, gpu, monkeypatch, scheme):
+    """V in host memory is refused before any entry point is asked (none is
+    reached here either way: the stand-in fails the test)."""
+    K, V = _kv(1, 2, 33, 128, "head", gpu)
+
+    def asked(name, *args):
+        pytest.fail(f"{name} was given a host pointer")
+
+    monkeypatch.setattr(pkg._lib, "call_if_built", asked)
+    with pytest.raises(ValueError, match="GPU"):
+        pkg.rs.forward_encode_kv(K, V.cpu(), 6, 2, scheme=scheme)
