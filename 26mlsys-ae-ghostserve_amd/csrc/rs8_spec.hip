@@ -382,9 +382,10 @@ extern "C" int kvec_rs8_decode(void* const* shards, int k, int m, int64_t shard_
 }
 
 // The packed rows and the stream of rs.forward_encode_kv / backwards_decode_kv
-// with these codes, or EUNSUPPORTED.
+// with these codes, or EUNSUPPORTED.  The encode only reads K and V, which may
+// then be the same memory.
 static int rs8_kv_stream(KvStream* s, const void* K, const void* V, int64_t half, const void* shards, int k, int m,
-                         int64_t S, const char* fn) {
+                         int64_t S, bool encode, const char* fn) {
     bool flat = false;
     if (m < 1 || S < 16 || !aligned16(shards) || half < 16 || uint64_t(k + m) * uint64_t(S) >= (uint64_t(1) << 31) ||
         S >= (int64_t(1) << 31) || !make_kv_stream(s, &flat, K, V, KvDims{1, 1, 1, half, 0, 0, 0}) ||
@@ -392,7 +393,7 @@ static int rs8_kv_stream(KvStream* s, const void* K, const void* V, int64_t half
         return set_error(KVEC_EUNSUPPORTED, "%s: layout or stripe not built", fn);
     if (!K || !V) return set_error(KVEC_EINVAL, "%s: null K or V", fn);
     const Span w[3] = {{shards, uint64_t(k + m) * uint64_t(S), "shards", -1}, {K, s->kb, "K", -1}, {V, s->kb, "V", -1}};
-    return check_no_alias(w, 3, nullptr, 0, fn);
+    return encode ? check_no_alias(w, 1, w + 1, 2, fn) : check_no_alias(w, 3, nullptr, 0, fn);
 }
 
 extern "C" int kvec_rs8_encode_kv(const void* key_input, const void* value_input, int64_t kv_half_bytes, void* shards,
@@ -404,7 +405,7 @@ extern "C" int kvec_rs8_encode_kv(const void* key_input, const void* value_input
     if (!shards) return set_error(KVEC_EINVAL, "%s: null pointer", fn);
     Rs8Io<kEncode> io{};
     if (m > 4) return set_error(KVEC_EUNSUPPORTED, "%s: %d parity rows", fn, m);
-    if ((rc = rs8_kv_stream(&io.kv, key_input, value_input, kv_half_bytes, shards, k, m, row_bytes, fn))) return rc;
+    if ((rc = rs8_kv_stream(&io.kv, key_input, value_input, kv_half_bytes, shards, k, m, row_bytes, true, fn))) return rc;
     io.sh = (uint8_t*)shards;
     io.k = k;
     uint8_t C[kRs8MaxM * kRs8MaxK];
@@ -433,7 +434,7 @@ extern "C" int kvec_rs8_recover_kv(void* shards, void* key_output, void* value_o
     if (ne > m) return set_error(KVEC_EDECODE, "%s: %d erasures > m=%d", fn, ne, m);
     Rs8Io<kDecode> io{};
     if (ne < 1 || ne > 4) return set_error(KVEC_EUNSUPPORTED, "%s: %d erasures", fn, ne);
-    if ((rc = rs8_kv_stream(&io.kv, key_output, value_output, kv_half_bytes, shards, k, m, row_bytes, fn))) return rc;
+    if ((rc = rs8_kv_stream(&io.kv, key_output, value_output, kv_half_bytes, shards, k, m, row_bytes, false, fn))) return rc;
     int surv[kRs8MaxK], outs[kRs8MaxM], no = 0;
     uint8_t M[kRs8MaxM * kRs8MaxK];
     if (!rs8_decode_rows(k, m, er, surv, outs, &no, M))

@@ -268,3 +268,18 @@ def test_rs_encode_refuses_host_values(pkg, gpu, monkeypatch, scheme):
     monkeypatch.setattr(pkg._lib, "call_if_built", asked)
     with pytest.raises(ValueError, match="GPU"):
         pkg.rs.forward_encode_kv(K, V.cpu(), 6, 2, scheme=scheme)
+
+
+@pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
+def test_rs_encode_of_shared_memory(pkg, gpu, scheme):
+    """K and V are only read: the same tensor, or two views of one buffer that
+    overlap, code like copies of them."""
+    buf = torch.randint(-32768, 32768, (3 * 33 * 128,), dtype=torch.int16, device=gpu).view(torch.float16)
+    K = buf[:2 * 33 * 128].view(1, 2, 33, 128)
+    for V in (K, buf[33 * 128:].view(1, 2, 33, 128)):
+        got, meta = pkg.rs.forward_encode_kv(K, V, 6, 2, scheme=scheme)
+        want, _ = pkg.rs.forward_encode_kv(K.clone(), V.clone(), 6, 2, scheme=scheme)
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        k2, v2 = pkg.rs.backwards_decode_kv(got, meta, [0, 3])
+        assert torch.equal(k2.view(torch.int16), K.view(torch.int16))
+        assert torch.equal(v2.view(torch.int16), V.view(torch.int16))
