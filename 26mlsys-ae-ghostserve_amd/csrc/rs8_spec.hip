@@ -105,6 +105,7 @@ template <int NOUT, int V, Rs8Mode MODE>
 __global__ __launch_bounds__(kRs8LoopBS) void gf8_loop_kernel(Rs8Io<MODE> io, Gf8Mix mix, int nin, int nout,
                                                               uint32_t S) {
     constexpr uint32_t TB = 16 * kRs8LoopBS * V, WB = 1024 * V;
+    static_assert((TB & (TB - 1)) == 0, "columns of the last tile stay below 2^32");
     __shared__ __attribute__((aligned(16))) uint32_t tab[kRs8MaxK][NOUT][6];   // nin is even or padded
     const int o0 = int(blockIdx.y) * NOUT, nj = (nin + 1) & ~1;
     for (int e = threadIdx.x; e < nj * NOUT * 6; e += kRs8LoopBS) {
@@ -114,6 +115,7 @@ __global__ __launch_bounds__(kRs8LoopBS) void gf8_loop_kernel(Rs8Io<MODE> io, Gf
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t t0 = blockIdx.x * TB;
     const uint32_t wb = t0 + uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6))) * WB;
+    // shards of up to 4 GiB: the tile divides 2^32, so a column never wraps
     auto col = [&](int v) { return wb + v * 1024 + 16 * lane; };
     __amdgpu_buffer_rsrc_t rs;
     if constexpr (MODE == kDecode) rs = chunk_rsrc(io.sh, io.sh_bytes);
@@ -226,7 +228,9 @@ static int launch_loop(const Rs8Io<MODE>& io, const Gf8Mix& mix, int nin, int no
     return check_launch(what);
 }
 
-// Shards of 2 GiB and more: one output at a time, inputs re-read through L2.
+// Shards of 4 GiB and more, past the loop kernel's 32-bit columns: one output at
+// a time, inputs re-read through L2 (shards of 2 GiB, this against the loop: RS(8,
+// 2) 5.2 against 3.4 ms, (10, 4) 12.0 against 5.0).
 __global__ __launch_bounds__(kRs8BS) void gf8_mix_generic_kernel(Ptrs<kRs8MaxK> in,
                                                                  Ptrs<kRs8MaxM> out, Gf8Mix mix,
                                                                  int nin, int nout, uint64_t nvec) {
@@ -284,7 +288,7 @@ static int launch_mix(uint8_t* const* in, int nin, uint8_t* const* out, int nout
         const uint32_t nvec = uint32_t(S / 16);
         hipLaunchKernelGGL(fn, dim3(blocks_for(nvec, kRs8BS * 2)), dim3(kRs8BS), 0, st, pi, po, mix,
                            uint32_t(S), nvec);
-    } else if (S < (int64_t(1) << 31)) {
+    } else if (fits_buffer(uint64_t(S))) {   // 32-bit columns
         return launch_loop<kShards>(Rs8Io<kShards>{pi, po}, mix, nin, nout, uint32_t(S), st, what);
     } else {
         const uint64_t nvec = uint64_t(S) / 16;

@@ -165,3 +165,37 @@ def test_chain_decode_every_pattern(pkg, ora, gpu, p, ks, R, unit):
                 sh[e].fill_(0x5A)
             pkg.spec.rdp_decode(sh, p, list(pat), unit_bytes=unit)
             assert all(torch.equal(a, b) for a, b in zip(sh, want)), (k, pat)
+
+
+@pytest.mark.parametrize("k,m,S", [(1, 1, 1 << 31), (3, 4, (1 << 31) + 4112), (2, 1, (1 << 32) - 16),
+                                   (1, 3, (1 << 32) - 16),
+                                   # past 32-bit columns: the other kernel
+                                   (1, 1, (1 << 32) + 16), (3, 2, (1 << 32) + 4112), (6, 2, 1 << 32)])
+def test_rs8_shards_of_gigabytes(pkg, ora, gpu, k, m, S):
+    """GF(2^8) shards up to and past 4 GiB: the parity at both ends and around
+    2 GiB against the oracle, decodes compared byte by byte."""
+    free, _ = torch.cuda.mem_get_info(gpu)
+    if free < (k + 2 * m + 1) * S + (8 << 30):
+        pytest.skip(f"needs {((k + 2 * m + 1) * S) >> 30} GiB of free device memory")
+    sh = [torch.empty(S, dtype=torch.uint8, device=gpu) for _ in range(k + m)]
+    try:
+        for t in sh:
+            t.view(torch.int64).random_()
+        pkg.spec.rs8_encode(sh[:k], sh[k:])
+        n = 16 * 1024
+        at = sorted({0, S - n, min(S, 1 << 31) - n, (1 << 31) - 4096 if S > (1 << 31) + n else 0})
+        cols = [np.concatenate([t[a:a + n].cpu().numpy() for a in at]) for t in sh]
+        want = ora.rs8_encode(cols[:k], m)
+        assert all(np.array_equal(c, np.asarray(w).reshape(-1)) for c, w in zip(cols[k:], want))
+        if k == 1 and m == 1:   # its one coefficient is 1 / (1 ^ 0)
+            assert torch.equal(sh[0], sh[1])
+        for er in ([0], list(range(k + m - m, k + m)), list(range(min(k, m)))):
+            keep = [sh[e].clone() for e in er]
+            for e in er:
+                sh[e].zero_()
+            pkg.spec.rs8_decode(sh, k, er)
+            assert all(torch.equal(sh[e], w) for e, w in zip(er, keep)), er
+            del keep
+    finally:
+        del sh
+        torch.cuda.empty_cache()
