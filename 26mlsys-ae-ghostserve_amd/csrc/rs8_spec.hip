@@ -254,21 +254,32 @@ __global__ __launch_bounds__(kRs8BS) void gf8_mix_generic_kernel(Ptrs<kRs8MaxK> 
 
 typedef void (*MixFn)(Ptrs<kRs8MaxK>, Ptrs<kRs8MaxM>, Gf8Mix, uint32_t, uint32_t);
 
-// Two outputs of four to six inputs keep the straight-line kernel from 60 MiB
-// shards on (512 MiB stream: RS(4, 2) 127-129 against 136 us for the loop, (5,
-// 2) 123 against 125, (6, 2) 115.5 against 118.4).  Below that (201 MB: (4, 2)
-// 53 against 51 us, (6, 2) 47.0 against 46.5) and on the other shapes that had
-// one the loop is as fast or faster: at 201 MB (4, 1) 43.5 against 42.7 us, (5,
-// 3) 56.1 against 55.0, (8, 2) 47.0 against 42.6, (10, 4) 57.2 against 50.7; at
-// 512 MiB (5, 3) 141 against 138, (8, 2) 112 against 114, (10, 4) 143 against 128.
-constexpr uint64_t kRs8StraightBytes = 60u << 20;
-static MixFn mix_fn(int nin, int nout, uint64_t S) {
-    if (nout != 2 || S < kRs8StraightBytes || !fits_buffer(S)) return nullptr;
+// Large shards of some shapes keep the straight-line kernel: two outputs of four
+// to six inputs from 60 MiB on (512 MiB stream: RS(4, 2) 127-129 against 136 us
+// for the loop, (5, 2) 123 against 125, (6, 2) 115.5 against 118.4; 201 MB: (4, 2)
+// 53 against 51 us, (6, 2) 47.0 against 46.5), two outputs of eight from 40 MiB
+// (shards of 34 MB 57-59 against 56-57 us, 42 MB 69 against 71, 55 MB 88 against 93,
+// 64 MiB 106 against 113-119, 201 MB 315 against 351, 805 MB 1293 against 1350), one
+// of ten from 48 MiB (42 MB 78 against 76, 59 MB 105 against 108, 134 MB 242
+// against 250).  On the other shapes that had one the loop is as fast or faster,
+// 1 MB to 2 GiB shards: (4, 1), (5, 1), (6, 1), (8, 1) and (5, 3) within 2 % from 34
+// MB on, (10, 2) of 20 MB 48 against 42 us and of 54 MB 115 against 111, (10, 4) of
+// 54 MB 128 against 122.
+struct MixKern {
+    MixFn fn;
+    int vec;   // 16-byte windows of a thread
+};
+static MixKern mix_kern(int nin, int nout, uint64_t S) {
+    const MixKern none = {nullptr, 0};
+    if (!fits_buffer(S) || S < (nin == 8 ? 40u << 20 : nin == 10 ? 48u << 20 : 60u << 20)) return none;
+    if (nout == 1 && nin == 10) return {&gf8_mix_kernel<10, 1, 2>, 2};
+    if (nout != 2) return none;
     switch (nin) {
-        case 4: return &gf8_mix_kernel<4, 2, 2>;
-        case 5: return &gf8_mix_kernel<5, 2, 2>;
-        case 6: return &gf8_mix_kernel<6, 2, 2>;
-        default: return nullptr;
+        case 4: return {&gf8_mix_kernel<4, 2, 2>, 2};
+        case 5: return {&gf8_mix_kernel<5, 2, 2>, 2};
+        case 6: return {&gf8_mix_kernel<6, 2, 2>, 2};
+        case 8: return {&gf8_mix_kernel<8, 2, 1>, 1};
+        default: return none;
     }
 }
 
@@ -284,9 +295,9 @@ static int launch_mix(uint8_t* const* in, int nin, uint8_t* const* out, int nout
         for (int j = 0; j < nin; ++j) perm_tables(M[o * nin + j], mix.t[o * nin + j]);
     }
     if (S == 0 || nout == 0) return KVEC_OK;
-    if (MixFn fn = mix_fn(nin, nout, uint64_t(S))) {
+    if (const MixKern kern = mix_kern(nin, nout, uint64_t(S)); kern.fn) {
         const uint32_t nvec = uint32_t(S / 16);
-        hipLaunchKernelGGL(fn, dim3(blocks_for(nvec, kRs8BS * 2)), dim3(kRs8BS), 0, st, pi, po, mix,
+        hipLaunchKernelGGL(kern.fn, dim3(blocks_for(nvec, kRs8BS * kern.vec)), dim3(kRs8BS), 0, st, pi, po, mix,
                            uint32_t(S), nvec);
     } else if (fits_buffer(uint64_t(S))) {   // 32-bit columns
         return launch_loop<kShards>(Rs8Io<kShards>{pi, po}, mix, nin, nout, uint32_t(S), st, what);

@@ -180,6 +180,25 @@ def test_rs8_straight_line_sizes(pkg, ora, gpu, k, S):
     assert torch.equal(data[0], full[0]) and torch.equal(data[1], full[1])
 
 
+# the same of the other shapes coded straight-line, one window a thread (8, 2)
+# and two
+@pytest.mark.parametrize("k,m,S", [(k, m, (mib << 20) + d) for k, m, mib in ((8, 2, 40), (10, 1, 48))
+                                   for d in (-16, 0, 1040)])
+def test_rs8_straight_line_wide(pkg, ora, gpu, k, m, S):
+    g = torch.Generator(device=gpu).manual_seed(k)
+    data = [torch.randint(-2**62, 2**62, (S // 8,), generator=g, device=gpu).view(torch.uint8) for _ in range(k)]
+    par = [torch.empty_like(d) for d in data[:m]]
+    pkg.spec.rs8_encode(data, par)
+    at = torch.cat([torch.arange(0, 16 * 1024), torch.arange(S - 16 * 1024, S)]).to(gpu)
+    want = ora.rs8_encode([d[at].cpu().numpy() for d in data], m)
+    assert all(np.array_equal(p[at].cpu().numpy(), np.asarray(w).reshape(-1)) for p, w in zip(par, want))
+    full = [d.clone() for d in data[:m]]
+    for d in data[:m]:
+        d.zero_()
+    pkg.spec.rs8_decode(data + par, k, list(range(m)))
+    assert all(torch.equal(a, b) for a, b in zip(data, full))
+
+
 # P and Q of rows in place, nine to sixteen of them: every word alignment of the
 # tensor, rows of exactly a tile, odd lengths, star words in the wrapped part
 @pytest.mark.parametrize("nd", range(9, 17))
