@@ -135,8 +135,9 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // First the syndromes, as the encode folds its parities: row[r] is the XOR of
 // row r's surviving cells (P's included), diag[d] that of diagonal d's and of
 // Q[d].  Lost shards are read through an empty buffer resource (zeros, no
-// memory traffic), so nothing here depends on the pattern and every diagonal
-// is a compile-time accumulator; the cells of rdp_group(p, k) shards are kept in
+// memory traffic), and so are the cells of diagonal p-1 when Q alone is lost,
+// which needs no row syndrome; nothing else here depends on the pattern and
+// every diagonal is a compile-time accumulator; the cells of rdp_group(p, k) shards are kept in
 // flight, a shard's requested as an earlier one's are folded.  Then the lost cells, from the syndromes in LDS (each lane its
 // own column, no barrier), at offsets that follow from c0 and c1:
 //   two columns   the chains of the paper (FAST 2004, section 4): from the
@@ -169,25 +170,30 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const RdpWave w = rdp_wave(geo, ROWS, blockIdx.x, threadIdx.x);
     if (w.within >= w.g) return;
     const uint32_t off = uint32_t(w.base) + w.within, g = uint32_t(w.g);
+    auto column = [](int s) { return s == K ? P - 1 : s; };
     {
         RdpAcc<P> row[ROWS], diag[ROWS];
         u32x4 x[G][ROWS];
         auto load = [&](int s) {
             // (offsets in the VGPR and soffset 0: the range check of an empty
             // resource must see the whole offset)
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                    sh.p[s], (short)0, int((lost.absent >> s) & 1 ? 0u : nb), int(kBufWord3));
+            auto view = [&](bool none) {
+                return __builtin_amdgcn_make_buffer_rsrc(sh.p[s], (short)0, int(none ? 0u : nb), int(kBufWord3));
+            };
+            const bool none = (lost.absent >> s) & 1;
+            const __amdgpu_buffer_rsrc_t rs = view(none), ro = view(none || lost.c0 < 0);
 #pragma unroll
             for (int r = 0; r < ROWS; ++r)
                 x[s % G][r] = __builtin_bit_cast(
-                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, off + r * g, 0, kAuxLoadNT));
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128((r + column(s)) % P == P - 1 ? ro : rs, off + r * g,
+                                                                     0, kAuxLoadNT));
         };
 #pragma unroll
         for (int s = 0; s < G; ++s) load(s);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < N; ++s) {
-            const int col = s == K ? P - 1 : s;
+            const int col = column(s);
 #pragma unroll
             for (int r = 0; r < ROWS; ++r) {
                 const int d = s == K + 1 ? r : (r + col) % P;
