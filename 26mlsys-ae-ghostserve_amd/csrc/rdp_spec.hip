@@ -162,7 +162,7 @@ struct RdpLoss {
 
 __device__ __forceinline__ void pin(u32x4& v) { asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w)); }
 
-template <int P, int K>
+template <int P, int K, bool NT>
 __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) void rdp_decode_chain_kernel(
         RdpPtrs sh, RdpLoss lost, RdpGeom geo, uint32_t nb) {
     constexpr int ROWS = P - 1, N = K + 2, G = rdp_group(P, N);
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
             for (int r = 0; r < ROWS; ++r)
                 x[s % G][r] = __builtin_bit_cast(
                         u32x4, __builtin_amdgcn_raw_buffer_load_b128((r + column(s)) % P == P - 1 ? ro : rs, off + r * g,
-                                                                     0, kAuxLoadNT));
+                                                                     0, NT ? kAuxLoadNT : 0));
         };
 #pragma unroll
         for (int s = 0; s < G; ++s) load(s);
@@ -255,24 +255,33 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
         }
 }
 
+// Non-temporal loads from stripe sets of more than 256 MiB on, ordinary ones up
+// to there: a set that fits the 256 MB memory-side cache is often still in it,
+// and non-temporal loads pass it by (three sets in turn; p = 5, k = 2, row planes,
+// two lost: set of 96 MiB 16 against 21 us, 128 MiB 21 against 31, where the map
+// below takes 23.5; 200 MiB equal; 400 MiB 69 against 66, 1 GiB 173 against 164).  Past p = 7
+// there are only the non-temporal ones.
+constexpr uint64_t kRdpCachedBytes = 256u << 20;
+
 typedef void (*ChainFn)(RdpPtrs, RdpLoss, RdpGeom, uint32_t);
-template <int P, int K = 1>
+template <int P, bool NT, int K = 1>
 ChainFn pick_chain(int k) {
     // k = p - 1 up to p = 7 has the compiled networks
     if constexpr (K > (P <= 7 ? P - 2 : P - 1)) {
         return nullptr;
     } else {
-        if (k == K) return &rdp_decode_chain_kernel<P, K>;
-        return pick_chain<P, K + 1>(k);
+        if (k == K) return &rdp_decode_chain_kernel<P, K, NT>;
+        return pick_chain<P, NT, K + 1>(k);
     }
 }
-static ChainFn chain_fn(int p, int k) {
+static ChainFn chain_fn(int p, int k, uint64_t nb) {
+    const bool nt = uint64_t(k + 2) * nb > kRdpCachedBytes;
     switch (p) {
-        case 3: return pick_chain<3>(k);
-        case 5: return pick_chain<5>(k);
-        case 7: return pick_chain<7>(k);
-        case 11: return pick_chain<11>(k);
-        case 13: return pick_chain<13>(k);
+        case 3: return nt ? pick_chain<3, true>(k) : pick_chain<3, false>(k);
+        case 5: return nt ? pick_chain<5, true>(k) : pick_chain<5, false>(k);
+        case 7: return nt ? pick_chain<7, true>(k) : pick_chain<7, false>(k);
+        case 11: return pick_chain<11, true>(k);
+        case 13: return pick_chain<13, true>(k);
         default: return nullptr;
     }
 }
@@ -518,7 +527,7 @@ extern "C" int kvec_rdp_decode(void* const* shards, int k, int p, int64_t row_by
     const RdpGeom geo = make_rdp_geom(uint64_t(row_bytes), uint64_t(unit_bytes));
     const dim3 grid(unsigned(rdp_waves(geo))), block(kBS);
     DecFn fn = decode_fn(p, k, a, b, fits_buffer(nb));
-    const ChainFn cfn = fits_buffer(nb) ? chain_fn(p, k) : nullptr;
+    const ChainFn cfn = fits_buffer(nb) ? chain_fn(p, k, nb) : nullptr;
     if (fn) {
         hipLaunchKernelGGL(fn, grid, block, 0, as_stream(stream), s, geo, nb);
     } else if (cfn) {

@@ -199,3 +199,47 @@ def test_rs8_shards_of_gigabytes(pkg, ora, gpu, k, m, S):
     finally:
         del sh
         torch.cuda.empty_cache()
+
+
+def _every_pattern(pkg, ora, gpu, p, k, R, unit):
+    """The encode at the ends of the shards against the oracle, and for every
+    pattern of one and two lost shards the rebuilt ones byte by byte."""
+    nb = (p - 1) * R
+    free, _ = torch.cuda.mem_get_info(gpu)
+    if free < (k + 5) * nb + (8 << 30):
+        pytest.skip(f"needs {((k + 5) * nb) >> 30} GiB of free device memory")
+    sh = [torch.empty(nb, dtype=torch.uint8, device=gpu) for _ in range(k + 2)]
+    try:
+        for t in sh[:k]:
+            t.view(torch.int64).random_()
+        pkg.spec.rdp_encode(sh[:k], sh[k], sh[k + 1], p=p, unit_bytes=unit)
+        # bytes of the shards that make whole codes: the first and the last stripe
+        # (of R mod unit, or unit, bytes a row), or both ends of the row planes
+        if unit:
+            g = R % unit or unit
+            at = [torch.arange(0, (p - 1) * unit), torch.arange(nb - (p - 1) * g, nb)]
+        else:
+            at = [(torch.arange(p - 1)[:, None] * R + x[None, :]).reshape(-1)
+                  for x in (torch.arange(0, 1024), torch.arange(R - 1024, R))]
+        for idx in at:
+            cols = [t[idx.to(gpu)].cpu().numpy() for t in sh]
+            Pw, Qw = ora.rdp_encode(cols[:k], p)
+            assert np.array_equal(cols[k], Pw.reshape(-1)) and np.array_equal(cols[k + 1], Qw.reshape(-1))
+        for pat in [(a,) for a in range(k + 2)] + list(itertools.combinations(range(k + 2), 2)):
+            keep = [sh[e].clone() for e in pat]
+            for e in pat:
+                sh[e].fill_(0x5A)
+            pkg.spec.rdp_decode(sh, p, list(pat), unit_bytes=unit)
+            assert all(torch.equal(sh[e], w) for e, w in zip(pat, keep)), pat
+            del keep
+    finally:
+        del sh
+        torch.cuda.empty_cache()
+
+
+# both sides of the size from which the chain decode loads past the caches
+@pytest.mark.parametrize("p,k", [(3, 1), (5, 1), (5, 3), (7, 2), (7, 5)])
+@pytest.mark.parametrize("unit", [0, 65536])
+@pytest.mark.parametrize("past", [0, 16])
+def test_chain_decode_large_sets(pkg, ora, gpu, p, k, unit, past):
+    _every_pattern(pkg, ora, gpu, p, k, (256 << 20) // ((k + 2) * (p - 1)) // 16 * 16 + past, unit)
