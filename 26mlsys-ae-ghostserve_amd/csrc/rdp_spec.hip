@@ -153,7 +153,8 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // byte-identical): 8 shards, two lost 43 us (5.8 TB/s) against 79; 10 shards 41
 // against 77; 12 shards and P lost 40 against 104; 5 shards (p = 7) 48 against
 // 59; 3 shards, one lost 54 against 56; a 1 MB stream of 8 shards 11.6 against
-// 43.  Lost shards of 4 GiB and more, past a buffer resource, keep that map.
+// 43.  Shards of 4 GiB and more, past a buffer resource, keep that map, and so
+// does generic_is_faster().
 struct RdpLoss {
     int c0, c1;        // lost columns (data shard, or p-1 for P), c0 < c1; -1: none
     int q;             // Q lost
@@ -299,6 +300,15 @@ static RdpLoss rdp_loss(int p, int k, int a, int b) {
     return l;
 }
 
+// Whether the generic kernel below is the faster one: p = 3 (one data shard and
+// its two parities), data or P lost along with Q, sets past the caches.  A lane
+// there loads two cells and stores four, and the way through LDS shows (two sets
+// in turn, against the chain kernel: set of 144 MiB 24 against 19-20 us, 300 MiB 52-55
+// against 53-57, 603 MiB 99-103 against 106-110, 1.5 GiB 248-267 against 258-282).
+static bool generic_is_faster(int p, int k, const RdpLoss& l, uint64_t nb) {
+    return p == 3 && l.q && l.c0 >= 0 && uint64_t(k + 2) * nb > kRdpCachedBytes;
+}
+
 // The decode map by input cell, for the generic kernel: each cell the outputs
 // need, with the set of outputs (bit o) that XOR it in.  Built on the host
 // from the plan's per-output masks.
@@ -327,8 +337,8 @@ inline RdpCellMap rdp_cell_map(const RdpPlan& plan) {
     return cm;
 }
 
-// Same map for any (p, k) and any shard size: today shards of 4 GiB and more
-// of the codes without a compiled network.  Each needed cell is loaded
+// Same map for any (p, k) and any shard size: today shards of 4 GiB and more of
+// the codes without a compiled network, and generic_is_faster().  Each needed cell is loaded
 // once, BATCH at a time so that BATCH are in flight, and folded into every
 // output that uses it (wave-uniform tests of its output set); the 2 ROWS
 // outputs accumulate in registers.  Sized per p, so that small codes keep
@@ -434,7 +444,8 @@ DecFn pick_decode(int e0, int e1) {
 
 // Compile-time XOR networks are built for the full-width codes p = 3, 5, 7,
 // through buffer resources (shards below 4 GiB) or flat addresses (larger); the
-// other codes take the chain kernel below 4 GiB and the generic one above.
+// other codes take the chain kernel below 4 GiB, but for generic_is_faster(), and
+// the generic one above.
 template <bool BUF>
 static DecFn decode_fn_t(int p, int k, int e0, int e1) {
     if (p == 7 && k == 6) return pick_decode<7, 6, BUF>(e0, e1);
@@ -527,11 +538,12 @@ extern "C" int kvec_rdp_decode(void* const* shards, int k, int p, int64_t row_by
     const RdpGeom geo = make_rdp_geom(uint64_t(row_bytes), uint64_t(unit_bytes));
     const dim3 grid(unsigned(rdp_waves(geo))), block(kBS);
     DecFn fn = decode_fn(p, k, a, b, fits_buffer(nb));
-    const ChainFn cfn = fits_buffer(nb) ? chain_fn(p, k, nb) : nullptr;
+    const RdpLoss loss = rdp_loss(p, k, a, b);
+    const ChainFn cfn = fits_buffer(nb) && !generic_is_faster(p, k, loss, nb) ? chain_fn(p, k, nb) : nullptr;
     if (fn) {
         hipLaunchKernelGGL(fn, grid, block, 0, as_stream(stream), s, geo, nb);
     } else if (cfn) {
-        hipLaunchKernelGGL(cfn, grid, block, 0, as_stream(stream), s, rdp_loss(p, k, a, b), geo, uint32_t(nb));
+        hipLaunchKernelGGL(cfn, grid, block, 0, as_stream(stream), s, loss, geo, uint32_t(nb));
     } else {
         RdpPlan plan = make_rdp_plan(p, k, a, b);
         if (!plan.ok)

@@ -243,3 +243,12 @@ def _every_pattern(pkg, ora, gpu, p, k, R, unit):
 @pytest.mark.parametrize("past", [0, 16])
 def test_chain_decode_large_sets(pkg, ora, gpu, p, k, unit, past):
     _every_pattern(pkg, ora, gpu, p, k, (256 << 20) // ((k + 2) * (p - 1)) // 16 * 16 + past, unit)
+
+
+# shards of 4 GiB and more, which the codes without a compiled network decode by
+# the general map (p = 3 past the caches, above, does so for two of its patterns)
+@pytest.mark.parametrize("p,k,R", [(3, 1, (1 << 31) + 1040), (5, 2, (1 << 30) + 16), (7, 3, 715_827_904),
+                                   (11, 1, 429_496_736), (13, 2, 357_913_952)])
+@pytest.mark.parametrize("unit", [0, 65536])
+def test_rdp_decode_by_the_map(pkg, ora, gpu, p, k, R, unit):
+    _every_pattern(pkg, ora, gpu, p, k, R, unit)
