@@ -787,6 +787,19 @@ GsParityFn gs_parity_fn(int nd) {
     }
 }
 
+// Whether the fused backup of nd rows gives way to the copy and the kernel of
+// 9 .. kGsMaxRows rows: up to the row length where the bytes that the copy moves
+// again outweigh the rows in flight.  Measured (K and V of 50 to 1600 MB): 9 rows
+// of 7.5 MB 39 us against 51 fused, 11.2 MB 56 against 55.5, 14.9 MB 77 against 69,
+// 186 MB 1026 against 708; 10 rows of 10 MB 57 against 63, 13.4 MB 77.5 against 75;
+// 12 rows of 16.8 MB 103 against 107, 22 MB 139 against 130.6; 16 rows of 12.6 MB 101
+// against 130, 16.8 MB 146 either way, 34 MB 284 against 225.  (So both are below
+// the row tensors of 2 GiB that the wide kernel takes.)
+static bool copy_then_wide(int nd, int64_t S) {
+    if (nd <= 8 || nd > kGsMaxRows || S < 64) return false;
+    return uint64_t(S) * 2 < (nd <= 10 ? 11u << 20 : 17u << 20);
+}
+
 static int gs_rdp_parity(uint16_t* sh, int nd, int64_t S, int star_base, hipStream_t st,
                          const char* what, const GsSource* fused = nullptr) {
     if (nd <= 0 || S <= 0) return KVEC_OK;  // the reference kernel returns at once
@@ -1020,9 +1033,9 @@ extern "C" int kvec_gs_rdp_backup(const void* K_TN, const void* V_TN, void* shar
         const uintptr_t R0 = uintptr_t(shards), Rend = R0 + (cap + 2 * uint64_t(S)) * 2;
         const uintptr_t Kp = uintptr_t(K_TN), Vp = uintptr_t(V_TN);
         const bool apart = (Kp + tn * 2 <= R0 || Kp >= Rend) && (Vp + tn * 2 <= R0 || Vp >= Rend);
-        // Nine to sixteen rows, which that kernel takes one at a time, are copied
-        // and then coded with every row in flight.
-        if (apart && (nd <= 8 || nd > kGsMaxRows || S < 64) && ((Kp ^ R0) & 15) == 0 && ((Vp ^ (R0 + tn * 2)) & 15) == 0) {
+        // Short rows, nine to sixteen of them, which that kernel takes one at a
+        // time, are copied and then coded with every row in flight.
+        if (apart && !copy_then_wide(nd, S) && ((Kp ^ R0) & 15) == 0 && ((Vp ^ (R0 + tn * 2)) & 15) == 0) {
             const uint64_t kv = 4 * tn, rows = 2 * cap;
             const GsSource g{(const uint8_t*)K_TN, (const uint8_t*)V_TN, int64_t(2 * tn),
                              int64_t(kv < rows ? kv : rows), int64_t(Rend - R0)};

@@ -302,3 +302,45 @@ def test_rs_encode_of_shared_memory(pkg, gpu, scheme):
         k2, v2 = pkg.rs.backwards_decode_kv(got, meta, [0, 3])
         assert torch.equal(k2.view(torch.int16), K.view(torch.int16))
         assert torch.equal(v2.view(torch.int16), V.view(torch.int16))
+
+
+def _packed_backup(pkg, gpu, nd, S, sb, tail):
+    """K, V and the row tensor of the packed backup of nd rows of S words, the
+    last `tail` of them padding (left as they were)."""
+    n = nd * S - tail
+    assert n % 16 == 0
+    K, V = (torch.empty(n // 2, dtype=torch.int16, device=gpu).random_() for _ in range(2))
+    sh = torch.zeros((nd + 2, S), dtype=torch.int16, device=gpu)
+    pkg.rdp.rdp_kernel.fused_backup_full_kv(K.view(torch.float16).view(1, -1), V.view(torch.float16).view(1, -1),
+                                            sh.view(torch.uint16), nd, S, 1, n // 2, sb)
+    return K, V, sh
+
+
+# both sides of the row length from which nine to sixteen rows are coded as they
+# are packed, in one launch
+@pytest.mark.parametrize("nd,S", [(9, (11 << 19) - 16), (9, 11 << 19), (10, (11 << 19) + 16), (11, (17 << 19) - 16),
+                                  (16, 17 << 19)])
+def test_packed_backup_row_lengths(pkg, ora, gpu, nd, S):
+    K, V, sh = _packed_backup(pkg, gpu, nd, S, 3, 16)
+    want = np.zeros((nd + 2, S), np.uint16)
+    ora.gs_pack(*(x.cpu().numpy().view(np.uint16).reshape(1, -1) for x in (K, V)), want, nd, S, 1, K.numel())
+    ora.gs_parity(want, nd, S, 3)
+    assert np.array_equal(sh.cpu().numpy().view(np.uint16), want)
+
+
+# a row tensor past 2 GiB
+@pytest.mark.parametrize("nd", [9, 16])
+def test_packed_backup_past_2gib(pkg, gpu, nd):
+    S = ((1 << 30) // (nd + 2) // 16 + 1) * 16
+    free, _ = torch.cuda.mem_get_info(gpu)
+    if free < 24 << 30:
+        pytest.skip("needs 24 GiB of free device memory")
+    K, V, sh = _packed_backup(pkg, gpu, nd, S, 5, 0)
+    assert torch.equal(sh[:nd].reshape(-1), torch.cat([K, V]))
+    P, Q = torch.zeros_like(sh[0]), torch.zeros_like(sh[0])
+    for r in range(nd):
+        P ^= sh[r]
+        x = torch.roll(sh[r], r)
+        x[(5 + r + r) % S] = 0   # the star word's diagonal
+        Q ^= x
+    assert torch.equal(sh[nd], P) and torch.equal(sh[nd + 1], Q)
