@@ -181,13 +181,15 @@ def call_if_built(name: str, *args) -> bool:
 
 def kv_bhtd(k, v):
     """The kvec_kv_bhtd of K and V tensors indexed [B, H, T, D], or None when
-    they differ in strides or a head's values are not adjacent."""
+    they differ in strides, a head's values are not adjacent, or heads or
+    tensors do not start and end on 16 bytes (no entry point takes those)."""
     B, H, T, D = k.shape
     ks, vs = k.stride(), v.stride()
-    if ks != vs or ks[3] != 1:
-        return None
     es = k.element_size()
-    return KvBhtd(k.data_ptr(), v.data_ptr(), B, H, T, D * es, ks[0] * es, ks[1] * es, ks[2] * es)
+    kp, vp = k.data_ptr(), v.data_ptr()
+    if ks != vs or ks[3] != 1 or (kp | vp | D * es) & 15:
+        return None
+    return KvBhtd(kp, vp, B, H, T, D * es, ks[0] * es, ks[1] * es, ks[2] * es)
 
 
 def ptr_array(tensors) -> C.Array:

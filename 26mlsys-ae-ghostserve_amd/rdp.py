@@ -123,33 +123,39 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
         shard_size, pad_words = spec_shard_size_words(total_words, nd, p)
     else:
         shard_size, pad_words = determine_shard_size_words(total_words, nd)
-    device = keys_bhtd.device
-    shards = torch.empty((nd + 2, shard_size), dtype=torch.uint16, device=device)
+    # one pass over K and V where they lie, when the layout allows it (what can
+    # be known here: up to twelve rows of 64 words and more); else token-major
+    # copies, then the pack and the code
+    kv = None
+    if scheme == "spec" or (nd <= 12 and shard_size >= 64):
+        kv = _lib.kv_bhtd(keys_bhtd, values_bhtd)
+    shards = torch.empty((nd + 2, shard_size), dtype=torch.uint16, device=keys_bhtd.device)
     t0 = torch.cuda.Event(enable_timing=True)
     t1 = torch.cuda.Event(enable_timing=True)
-    t0.record()
-    # one pass over K and V where they lie, when their layout allows it; else
-    # token-major copies, then the pack and the code
-    kv = _lib.kv_bhtd(keys_bhtd, values_bhtd)
-    if scheme == "spec":
-        if kv is None or not _lib.call_if_built("kvec_kv_pack_bhtd", kv, shards.data_ptr(),
-                                                2 * nd * int(shard_size), _stream(shards)):
-            K_TN, V_TN = _token_major(keys_bhtd, values_bhtd)
-            shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
-            t0.record()
-            _lib.call("kvec_rs16_pack", K_TN.data_ptr(), V_TN.data_ptr(), shards.data_ptr(),
-                      T * n, T * n, _stream(shards))
-        rows = _rows_u8(shards)
-        spec.rdp_encode(rows[:nd], rows[nd], rows[nd + 1], p, unit_bytes=spec.RDP_UNIT)
-    elif kv is None or not _lib.call_if_built("kvec_gs_rdp_backup_kv", kv, shards.data_ptr(), nd,
-                                              int(shard_size), int(star_base), _stream(shards)):
+    direct = False
+    if kv is not None:
+        t0.record()
+        if scheme == "spec":
+            direct = _lib.call_if_built("kvec_kv_pack_bhtd", kv, shards.data_ptr(),
+                                        2 * nd * int(shard_size), _stream(shards))
+        else:
+            direct = _lib.call_if_built("kvec_gs_rdp_backup_kv", kv, shards.data_ptr(), nd,
+                                        int(shard_size), int(star_base), _stream(shards))
+    if not direct:
         K_TN, V_TN = _token_major(keys_bhtd, values_bhtd)
         # the reference zero-fills everything; only the padding words are read
         # before being written
         shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
         t0.record()
-        rdp_kernel.fused_backup_full_kv(K_TN, V_TN, shards, nd, int(shard_size), int(T), int(n),
-                                        int(star_base))
+        if scheme == "spec":
+            _lib.call("kvec_rs16_pack", K_TN.data_ptr(), V_TN.data_ptr(), shards.data_ptr(),
+                      T * n, T * n, _stream(shards))
+        else:
+            rdp_kernel.fused_backup_full_kv(K_TN, V_TN, shards, nd, int(shard_size), int(T), int(n),
+                                            int(star_base))
+    if scheme == "spec":
+        rows = _rows_u8(shards)
+        spec.rdp_encode(rows[:nd], rows[nd], rows[nd + 1], p, unit_bytes=spec.RDP_UNIT)
     t1.record()
     torch.cuda.synchronize()
     backup_ms = t0.elapsed_time(t1)
@@ -182,26 +188,29 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
     B, H, _, D = pkg["shape_BHTD"]
     dtype = pkg.get("dtype", torch.float16)
 
-    kv_shape = (int(B), int(H), int(T), int(D))
-    keys = torch.empty(kv_shape, dtype=dtype, device=shards.device)
-    values = torch.empty(kv_shape, dtype=dtype, device=shards.device)
-    _lib.require_cuda(shards, keys, values, what="fused_recovery_full_kv tensor")
+    is_spec = pkg.get("scheme", "ghostserve") == "spec"
+    _lib.require_cuda(shards, what="fused_recovery_full_kv tensor")
+    # the rows written straight to K and V when the layout allows it (known
+    # before they are allocated: heads of whole 16 bytes, rows of 64 words and
+    # more); else through a token-major copy
+    kv = None
+    if D * dtype.itemsize % 16 == 0 and (is_spec or shard_size >= 64):
+        kv_shape = (int(B), int(H), int(T), int(D))
+        keys = torch.empty(kv_shape, dtype=dtype, device=shards.device)
+        values = torch.empty(kv_shape, dtype=dtype, device=shards.device)
+        kv = _lib.kv_bhtd(keys, values)
     t0 = torch.cuda.Event(enable_timing=True)
     t1 = torch.cuda.Event(enable_timing=True)
     t0.record()
-    # the rows written straight to K and V when the layout allows it; else
-    # through a token-major copy
-    kv = _lib.kv_bhtd(keys, values)
-    is_spec = pkg.get("scheme", "ghostserve") == "spec"
     if is_spec:
         lost = [int(e) for e in (missing_a, missing_b) if 0 <= int(e) < nd + 2]
         spec.rdp_decode(_rows_u8(shards), int(pkg["p"]), lost, unit_bytes=spec.RDP_UNIT)
-        direct = _lib.call_if_built("kvec_kv_unpack_bhtd", shards.data_ptr(),
-                                    2 * int(nd) * int(shard_size), kv, _stream(shards))
+        direct = kv is not None and _lib.call_if_built(
+            "kvec_kv_unpack_bhtd", shards.data_ptr(), 2 * int(nd) * int(shard_size), kv, _stream(shards))
     else:
-        direct = _lib.call_if_built("kvec_gs_rdp_recover_kv", shards.data_ptr(), kv, int(nd),
-                                    int(shard_size), int(star_base), int(missing_a),
-                                    int(missing_b), _stream(shards))
+        direct = kv is not None and _lib.call_if_built(
+            "kvec_gs_rdp_recover_kv", shards.data_ptr(), kv, int(nd), int(shard_size), int(star_base),
+            int(missing_a), int(missing_b), _stream(shards))
     if not direct:
         packed_TN = torch.empty(2 * T * n, dtype=dtype, device=shards.device)
         if is_spec:
@@ -213,10 +222,8 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
                                               int(missing_b))
     t1.record()
     if not direct:
-        dK = packed_TN[:T * n].view(T, n)
-        dV = packed_TN[T * n:].view(T, n)
-        keys.copy_(dK.view(T, B, H, D).permute(1, 2, 0, 3))
-        values.copy_(dV.view(T, B, H, D).permute(1, 2, 0, 3))
+        keys, values = (x.view(T, B, H, D).permute(1, 2, 0, 3).contiguous()
+                        for x in (packed_TN[:T * n], packed_TN[T * n:]))
     torch.cuda.synchronize()
     recover_ms = t0.elapsed_time(t1)
     return keys, values, {"recover_ms": recover_ms}

@@ -344,3 +344,22 @@ def test_packed_backup_past_2gib(pkg, gpu, nd):
         x[(5 + r + r) % S] = 0   # the star word's diagonal
         Q ^= x
     assert torch.equal(sh[nd], P) and torch.equal(sh[nd + 1], Q)
+
+
+@pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
+@pytest.mark.parametrize("B,H,T,D,order,nd", [(1, 8, 33, 20, "head", 5), (2, 2, 65, 12, "token", 5),
+                                              (1, 2, 33, 64, "odd", 5), (1, 1, 4, 20, "head", 5)])
+def test_copied_layouts_ask_no_entry_point(pkg, gpu, monkeypatch, scheme, B, H, T, D, order, nd):
+    """Layouts that no one-pass entry point takes go to the copies without
+    preparing for one: heads of no whole 16 bytes, and K and V off alignment
+    (whose recovery, into K and V of its own, is direct)."""
+    K, V = _kv(B, H, T, D, order, gpu)
+    asked = []
+    real = pkg._lib.call_if_built
+    monkeypatch.setattr(pkg._lib, "call_if_built", lambda name, *a: asked.append(name) or real(name, *a))
+    pk = pkg.rdp.fused_backup_full_kv(K, V, nd, scheme=scheme)
+    assert not asked
+    k2, v2, _ = pkg.rdp.fused_recovery_full_kv(pk, 1)
+    assert len(asked) == (order == "odd")
+    assert torch.equal(k2.view(torch.int16), K.view(torch.int16).contiguous())
+    assert torch.equal(v2.view(torch.int16), V.view(torch.int16).contiguous())
