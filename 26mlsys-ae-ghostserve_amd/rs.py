@@ -237,7 +237,7 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
     # and the layout allows it
     if (one_pass and missing_data and
             avail_par[:len(missing_data)] == list(range(len(missing_data)))):
-        lost = np.asarray(missing_data, dtype=np.int32)
+        lost = np.asarray([int(i) for i in missing_data], dtype=np.int32)
         if _lib.call_if_built("kvec_rs16_recover_kv", shards.data_ptr(), K.data_ptr(), V.data_ptr(),
                               2 * int(N_k), int(num_data), int(num_parity), int(shard_sz),
                               lost.ctypes.data, len(missing_data), _stream(shards)):

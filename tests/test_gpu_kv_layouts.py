@@ -363,3 +363,18 @@ def test_copied_layouts_ask_no_entry_point(pkg, gpu, monkeypatch, scheme, B, H, 
     assert len(asked) == (order == "odd")
     assert torch.equal(k2.view(torch.int16), K.view(torch.int16).contiguous())
     assert torch.equal(v2.view(torch.int16), V.view(torch.int16).contiguous())
+
+
+@pytest.mark.parametrize("as_given", [
+    lambda er, gpu: torch.tensor(er, device=gpu), lambda er, gpu: list(torch.tensor(er, device=gpu)),
+    lambda er, gpu: np.array(er), lambda er, gpu: tuple(er)], ids=["gpu tensor", "gpu scalars", "numpy", "tuple"])
+def test_rs16_lost_rows_as_given(pkg, gpu, as_given):
+    """The lost rows as a program may hold them."""
+    K, V = _kv(1, 2, 33, 128, "head", gpu)
+    sh, meta = pkg.rs.forward_encode_kv(K, V, 6, 2)
+    for er in ([3], [1, 4]):
+        for e in er:
+            sh.view(torch.int16)[e] = 0x5A5A
+        k2, v2 = pkg.rs.backwards_decode_kv(sh, meta, as_given(er, gpu))
+        assert torch.equal(k2.view(torch.int16), K.view(torch.int16)), er
+        assert torch.equal(v2.view(torch.int16), V.view(torch.int16)), er
