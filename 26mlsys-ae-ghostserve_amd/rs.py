@@ -219,10 +219,13 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
     V = torch.empty(N_v, dtype=dtype, device=device)
     one_pass = (N_k == N_v and shards.is_cuda and shards.is_contiguous() and
                 K.element_size() == 2 and shards.element_size() == 2)
+    # whole rows that the tensor has: a program may hand in one without the
+    # parity rows that it lost
+    rows_held = shards.numel() // shard_sz
     if is_spec:
         if missing_shards:
             lost = np.ascontiguousarray([int(i) for i in missing_shards], dtype=np.int32)
-            if (one_pass and lost.max() < num_data + num_parity
+            if (one_pass and rows_held == num_data + num_parity and lost.max() < rows_held
                     and _rows_in_range("spec", num_data, num_parity)
                     and _lib.call_if_built("kvec_rs8_recover_kv", shards.data_ptr(), K.data_ptr(),
                                            V.data_ptr(), 2 * int(N_k), int(num_data),
@@ -235,11 +238,12 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
         missing_data = []
     # the rebuild and the split in one pass when the first parity rows serve
     # and the layout allows it
-    if (one_pass and missing_data and
+    if (one_pass and missing_data and rows_held >= num_data + len(missing_data) and
             avail_par[:len(missing_data)] == list(range(len(missing_data)))):
         lost = np.asarray([int(i) for i in missing_data], dtype=np.int32)
         if _lib.call_if_built("kvec_rs16_recover_kv", shards.data_ptr(), K.data_ptr(), V.data_ptr(),
-                              2 * int(N_k), int(num_data), int(num_parity), int(shard_sz),
+                              2 * int(N_k), int(num_data),
+                              min(int(num_parity), rows_held - int(num_data)), int(shard_sz),
                               lost.ctypes.data, len(missing_data), _stream(shards)):
             return K.view(B, H, T, D), V.view(B, H, T, D)
     if missing_data:

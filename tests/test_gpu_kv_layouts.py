@@ -378,3 +378,38 @@ def test_rs16_lost_rows_as_given(pkg, gpu, as_given):
         k2, v2 = pkg.rs.backwards_decode_kv(sh, meta, as_given(er, gpu))
         assert torch.equal(k2.view(torch.int16), K.view(torch.int16)), er
         assert torch.equal(v2.view(torch.int16), V.view(torch.int16)), er
+
+
+def test_rs_decode_of_fewer_rows(pkg, gpu, monkeypatch):
+    """A shard tensor without all the parity rows: the one-pass decode is told
+    the rows that are there, or not asked.  (The stand-in launches nothing.)"""
+    K, V = _kv(1, 2, 33, 128, "head", gpu)
+    k, m = 6, 3
+
+    class Asked(Exception):
+        pass
+
+    def asked(name, *args):
+        raise Asked(name, args)
+
+    for scheme in ("ghostserve", "spec"):
+        sh, meta = pkg.rs.forward_encode_kv(K, V, k, m, scheme=scheme)
+        for rows, lost in ((k + 1, [2]), (k + 2, [0, 5])):
+            with monkeypatch.context() as mp:
+                mp.setattr(pkg._lib, "call_if_built", asked)
+                mp.setattr(pkg.spec, "rs8_decode", lambda *a: asked("general", *a))
+                # (the general decode of scheme "spec" refuses such a tensor when its
+                # bytes do not make k + m equal rows)
+                with pytest.raises((Asked, RuntimeError)) as e:
+                    pkg.rs.backwards_decode_kv(sh[:rows].clone(), meta, lost)
+            if scheme == "spec":
+                assert e.type is RuntimeError or e.value.args[0] == "general"
+            else:
+                name, args = e.value.args
+                assert name == "kvec_rs16_recover_kv" and args[4] + args[5] == rows
+                part = sh[:rows].clone()
+                part.view(torch.int16)[lost] = 0x5A5A
+                k2, v2 = pkg.rs.backwards_decode_kv(part, meta, lost)
+                assert torch.equal(part.view(torch.int16), sh[:rows].view(torch.int16))
+                assert torch.equal(k2.view(torch.int16), K.view(torch.int16))
+                assert torch.equal(v2.view(torch.int16), V.view(torch.int16))
