@@ -192,9 +192,9 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
     _lib.require_cuda(shards, what="fused_recovery_full_kv tensor")
     # the rows written straight to K and V when the layout allows it (known
     # before they are allocated: heads of whole 16 bytes, rows of 64 words and
-    # more); else through a token-major copy
+    # more); else, and where n is not the shape's, through a token-major copy
     kv = None
-    if D * dtype.itemsize % 16 == 0 and (is_spec or shard_size >= 64):
+    if D * dtype.itemsize % 16 == 0 and (is_spec or shard_size >= 64) and n == B * H * D:
         kv_shape = (int(B), int(H), int(T), int(D))
         keys = torch.empty(kv_shape, dtype=dtype, device=shards.device)
         values = torch.empty(kv_shape, dtype=dtype, device=shards.device)

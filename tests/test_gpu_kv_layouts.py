@@ -413,3 +413,13 @@ def test_rs_decode_of_fewer_rows(pkg, gpu, monkeypatch):
                 assert torch.equal(part.view(torch.int16), sh[:rows].view(torch.int16))
                 assert torch.equal(k2.view(torch.int16), K.view(torch.int16))
                 assert torch.equal(v2.view(torch.int16), V.view(torch.int16))
+
+
+@pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
+def test_rdp_recovery_refuses_other_shape(pkg, gpu, scheme):
+    """A package whose words a token are not its shape's."""
+    K, V = _kv(1, 4, 65, 64, "head", gpu)
+    pk = pkg.rdp.fused_backup_full_kv(K, V, 5, scheme=scheme)
+    for shape in ((1, 2, 65, 64), (1, 4, 65, 32)):
+        with pytest.raises(RuntimeError):
+            pkg.rdp.fused_recovery_full_kv(dict(pk, shape_BHTD=shape), 1)
