@@ -18,7 +18,8 @@ import torch  # noqa: F401  (must precede CDLL, see module docstring)
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libkvec.so")
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
+# torch's own accessor of a stream handle; not public, so maybe not there
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 _vp = C.c_void_p
 _i = C.c_int
@@ -200,7 +201,8 @@ def stream_handle(device) -> int:
     """hipStream_t of torch's current stream on ``device``.  For a GPU tensor's
     device it is read without building a Stream object: a small call is bound
     by its host time."""
-    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+    if (_raw_stream is not None and isinstance(device, torch.device) and device.type == "cuda"
+            and device.index is not None):
         return _raw_stream(device.index)
     return int(torch.cuda.current_stream(device).cuda_stream)
 

@@ -189,6 +189,23 @@ def test_product_fails_loudly_without_library(pkg, monkeypatch, tmp_path):
         pkg._lib.lib()
 
 
+def test_bindings_without_the_raw_stream(pkg, monkeypatch):
+    """A torch without the private stream accessor: the bindings import, and
+    the handle comes from the public Stream object."""
+    import importlib.util
+    import torch
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    spec = importlib.util.spec_from_file_location("_kvec_lib_t", pkg._lib.__file__)
+    lib = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(lib)
+
+    class Stream:
+        cuda_stream = 4711
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: Stream)
+    assert lib.stream_handle(torch.device("cuda:0")) == 4711
+
+
 def test_chunk_width(pkg):
     L = pkg._lib.lib()
     # 16 x 2048 tokens x 32 layers x 256 B records (fp8, 1 head x 128) over k=5, p=7
