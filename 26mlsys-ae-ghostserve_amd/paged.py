@@ -40,17 +40,16 @@ class PagedKV:
         self.heads, self.dim = H, D
         self._c = _lib.PagedKV(pool.data_ptr(), npages, L, self.token_bytes, pt,
                                page_table.data_ptr(), B, pps, self.tok_off, self.tokens)
-        self._bytes = None
 
     @property
     def c(self):
         return self._c
 
     def stream_bytes(self) -> int:
-        # the descriptor is fixed, and so is its stream
-        if self._bytes is None:
-            self._bytes = int(_lib.lib().kvec_kv_stream_bytes(self._c))
-        return self._bytes
+        # kvec_kv_stream_bytes from the descriptor as it is now (a program may
+        # have moved it on through .c), without the call
+        c = self._c
+        return c.layers * c.batch * c.tokens * 2 * c.token_bytes
 
     def stream_shape(self):
         return (self.layers, self.batch, self.tokens, 2, self.heads, self.dim)

@@ -103,3 +103,14 @@ def test_paged_encode_unbuilt_config_raises(pkg, gpu):
     torch.cuda.synchronize()
     assert bool((P == 0x55).all()) and bool((Q == 0x55).all())
     assert all(bool((d == 0x77).all()) for d in data)
+
+
+def test_stream_bytes_follow_the_descriptor(pkg, gpu):
+    """A descriptor moved on through .c (the next step's tokens): the stream's
+    size, which gather() allocates by, is the library's for it."""
+    pool = torch.zeros((2, 8, 16, 2, 2, 64), dtype=torch.bfloat16, device=gpu)
+    table = torch.arange(8, dtype=torch.int32, device=gpu).view(2, 4)
+    kv = pkg.paged.PagedKV(pool, table, 0, 5)
+    for tokens in (5, 17, 1, 64):
+        kv.c.tokens = tokens
+        assert kv.stream_bytes() == pkg._lib.lib().kvec_kv_stream_bytes(kv.c) == 2 * 2 * tokens * 2 * 256
