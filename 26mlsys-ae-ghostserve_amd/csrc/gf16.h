@@ -117,4 +117,7 @@ __device__ __forceinline__ void gf16_step_pow_xor(uint32_t (&a)[4], int e, const
     }
 }
 
+// Whether the pack and kvec_rs16_encode beat the one-pass encode, gs_rs16.hip.
+bool rs16_ring_encode_faster(int k, int m, uint64_t Sb);
+
 }  // namespace kvec

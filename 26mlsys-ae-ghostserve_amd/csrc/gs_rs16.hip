@@ -1892,6 +1892,28 @@ extern "C" int kvec_rs16_split(const void* in, void* k_out, void* v_out, int64_t
 
 // encode_rs_u16, benchmark/rs/kernel.cu:265-285: copy the data rows, then the
 // parity rows.  gf_exp / gf_log are the device tables of init_gf_tables().
+namespace kvec {
+// Whether the pack and then kvec_rs16_encode are faster than the one-pass
+// encode of gs_rs16_kv.hip: three or four parities of many short rows that are
+// whole ring tiles.  There the time is a wave's way through the rows, and the
+// ring kernel's step from row to row (two windows a thread, byte maps or
+// doublings) is the shorter one, 0.52 us with three parities and 0.7 with four
+// against 0.9 for bit planes.  Whole calls, pack and encode against one pass:
+// three parities, 64 rows of 64 KiB 40 against 56 us, 1 MiB 58 against 68, 2 MiB 81
+// against 76, 24 rows 22 either way; 256 rows of 256 KiB 153 against 240; four
+// parities, 64 rows of 64 KiB 53 against 58, 1 MiB 73 against 70, 40 rows of 64 KiB
+// 36 against 37, 32 rows 30 either way; 256 rows of 256 KiB 201 against 246.  A
+// partial last tile is one more launch for that path (64 rows of 4 KiB 63 and 78
+// us) and the one pass always the faster.
+bool rs16_ring_encode_faster(int k, int m, uint64_t Sb) {
+    constexpr uint64_t TB = 16 * kRsHBS * 2, KiB = 1024;
+    if (Sb % TB) return false;
+    if (m == 3) return k >= 28 && Sb < 1536 * KiB;
+    if (m == 4) return k >= 40 && Sb < (k >= 64 ? 1024 : 256) * KiB;
+    return false;
+}
+}  // namespace kvec
+
 extern "C" int kvec_rs16_encode(const void* data_padded, void* shards, int data_shards,
                                 int parity_shards, int shard_size, const uint16_t* gf_exp,
                                 const uint16_t* gf_log, void* stream) {

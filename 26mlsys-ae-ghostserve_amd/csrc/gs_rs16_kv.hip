@@ -592,7 +592,7 @@ extern "C" int kvec_rs16_encode_kv(const void* key_input, const void* value_inpu
     if (!kern.fn || data_shards < 1 || data_shards > 65535 || shard_size < 64 || !aligned16(shards) ||
         rows * Sb > (uint64_t(1) << 31) - 16 || kv_half_bytes < 16 ||
         !make_kv_stream(&s, &flat, key_input, value_input, KvDims{1, 1, 1, kv_half_bytes, 0, 0, 0}) ||
-        2 * uint64_t(s.kb) > uint64_t(data_shards) * Sb)
+        2 * uint64_t(s.kb) > uint64_t(data_shards) * Sb || rs16_ring_encode_faster(data_shards, parity_shards, Sb))
         return set_error(KVEC_EUNSUPPORTED, "%s: layout or stripe not built", fn);
     if (!key_input || !value_input) return set_error(KVEC_EINVAL, "%s: null K or V", fn);
     const Span w = {shards, rows * Sb, "shards", -1};

@@ -345,7 +345,8 @@ int kvec_rs16_encode(const void* data_padded, void* shards, int data_shards, int
  * of kvec_rs16_encode with the tables of kvec_gf16_tables.  Every byte of
  * shards is written.  KVEC_EUNSUPPORTED, with nothing enqueued, outside: 1 to 4
  * parity rows, K, V, shards and kv_half_bytes multiples of 16, shard_size >=
- * 64, K and V below 1 GiB, shards below 2 GiB. */
+ * 64, K and V below 1 GiB, shards below 2 GiB; and for three or four parities of
+ * many short rows of whole 8 KiB, where kvec_rs16_encode is the faster way. */
 int kvec_rs16_encode_kv(const void* key_input, const void* value_input, int64_t kv_half_bytes, void* shards,
                         int data_shards, int parity_shards, int shard_size, void* stream);
 /* reconstruct_rs_u16_inplace, :287-312: rebuild the m data rows listed in the

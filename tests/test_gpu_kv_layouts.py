@@ -423,3 +423,24 @@ def test_rdp_recovery_refuses_other_shape(pkg, gpu, scheme):
     for shape in ((1, 2, 65, 64), (1, 4, 65, 32)):
         with pytest.raises(RuntimeError):
             pkg.rdp.fused_recovery_full_kv(dict(pk, shape_BHTD=shape), 1)
+
+
+# three and four parities around the lines past which many short rows of whole
+# 8 KiB are packed and coded apart: (k, m, bytes of a row, one pass)
+@pytest.mark.parametrize("k,m,Sb,one_pass", [
+    (27, 3, 8192, True), (28, 3, 8192, False), (32, 3, 8192 + 16, True), (39, 4, 16384, True), (40, 4, 16384, False),
+    (40, 4, 256 << 10, True), (64, 4, 256 << 10, False), (64, 4, 1 << 20, True), (96, 3, (1 << 20) + 8192, False),
+    (30, 3, 1536 << 10, True), (64, 2, 8192, True)])
+def test_rs16_many_short_rows(pkg, ora, gpu, monkeypatch, k, m, Sb, one_pass):
+    T = k * Sb // 512   # K and V of one head of 128
+    K, V = _kv(1, 1, T, 128, "head", gpu, seed=k)
+    took = []
+    real = pkg._lib.call_if_built
+    monkeypatch.setattr(pkg._lib, "call_if_built", lambda name, *a: took.append(real(name, *a)) or took[-1])
+    sh, meta = pkg.rs.forward_encode_kv(K, V, k, m)
+    assert meta["shard_sz"] * 2 == Sb and took == [one_pass]
+    data = np.zeros(k * meta["shard_sz"], np.uint16)
+    flat = np.concatenate([x.view(torch.int16).cpu().numpy().reshape(-1).view(np.uint16) for x in (K, V)])
+    data[:flat.size] = flat
+    want = ora.rs16_encode(data, k, m, meta["shard_sz"], *pkg.rs.init_gf_tables())
+    assert np.array_equal(sh.cpu().numpy(), want)
