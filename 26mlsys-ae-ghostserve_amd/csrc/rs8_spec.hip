@@ -101,7 +101,7 @@ struct Rs8Io<kDecode> {
 
 constexpr int kRs8LoopBS = 256;
 
-template <int NOUT, int V, Rs8Mode MODE>
+template <int NOUT, int V, Rs8Mode MODE, bool NT = true>
 __global__ __launch_bounds__(kRs8LoopBS) void gf8_loop_kernel(Rs8Io<MODE> io, Gf8Mix mix, int nin, int nout,
                                                               uint32_t S) {
     constexpr uint32_t TB = 16 * kRs8LoopBS * V, WB = 1024 * V;
@@ -128,7 +128,11 @@ __global__ __launch_bounds__(kRs8LoopBS) void gf8_loop_kernel(Rs8Io<MODE> io, Gf
         if (j >= nin) return;   // uniform
         if constexpr (MODE == kShards) {
 #pragma unroll
-            for (int v = 0; v < V; ++v) x[v] = ld_stream(io.in.p[j], col(v) < S ? col(v) : 0u);
+            for (int v = 0; v < V; ++v) {
+                const uint8_t* p = io.in.p[j];
+                const uint32_t c = col(v) < S ? col(v) : 0u;
+                x[v] = NT ? ld_stream(p, c) : ld16(p + c);
+            }
         } else if constexpr (MODE == kDecode) {
             const uint32_t r0 = uint32_t(io.in[j]) * S;
 #pragma unroll
@@ -211,7 +215,7 @@ __global__ __launch_bounds__(kRs8LoopBS) void gf8_loop_kernel(Rs8Io<MODE> io, Gf
 // against 42).  Elsewhere one is faster: 134 MB of K and V in six rows, encode
 // 59 against 61 us, two lost 62 against 69, one lost 58 against 62; RS(10, 4) of
 // 67 MB 34 against 38.  128 and 512 threads: within 5 % either way.
-template <Rs8Mode MODE>
+template <Rs8Mode MODE, bool NT = true>
 static int launch_loop(const Rs8Io<MODE>& io, const Gf8Mix& mix, int nin, int nout, uint32_t S, hipStream_t st,
                        const char* what) {
     constexpr int W = MODE == kDecode ? 2 : 1;
@@ -220,17 +224,19 @@ static int launch_loop(const Rs8Io<MODE>& io, const Gf8Mix& mix, int nin, int no
                            io, mix, nin, nout, S);
     };
     switch (nout) {
-        case 1: go(&gf8_loop_kernel<1, 1, MODE>, 1, 1); break;
-        case 2: go(&gf8_loop_kernel<2, 1, MODE>, 2, 1); break;
-        case 3: go(&gf8_loop_kernel<3, W, MODE>, 3, W); break;
-        default: go(&gf8_loop_kernel<4, W, MODE>, 4, W); break;
+        case 1: go(&gf8_loop_kernel<1, 1, MODE, NT>, 1, 1); break;
+        case 2: go(&gf8_loop_kernel<2, 1, MODE, NT>, 2, 1); break;
+        case 3: go(&gf8_loop_kernel<3, W, MODE, NT>, 3, W); break;
+        default: go(&gf8_loop_kernel<4, W, MODE, NT>, 4, W); break;
     }
     return check_launch(what);
 }
 
-// Shards of 4 GiB and more, past the loop kernel's 32-bit columns: one output at
-// a time, inputs re-read through L2 (shards of 2 GiB, this against the loop: RS(8,
-// 2) 5.2 against 3.4 ms, (10, 4) 12.0 against 5.0).
+// One output at a time, inputs re-read through L2: one input and one output (shards
+// of 33 MB 11.0 us against 13.9 by the loop, which pairs inputs, 100 MB 33.4 against
+// 35.8, 201 MB 67.0 against 69.5), and shards of 4 GiB and more, past the loop
+// kernel's 32-bit columns (of 2 GiB, this against the loop: RS(8, 2) 5.2 against 3.4
+// ms, (10, 4) 12.0 against 5.0).
 __global__ __launch_bounds__(kRs8BS) void gf8_mix_generic_kernel(Ptrs<kRs8MaxK> in,
                                                                  Ptrs<kRs8MaxM> out, Gf8Mix mix,
                                                                  int nin, int nout, uint64_t nvec) {
@@ -283,6 +289,14 @@ static MixKern mix_kern(int nin, int nout, uint64_t S) {
     }
 }
 
+// The loop's loads from separate shards: ordinary ones up to 128 MiB of inputs and
+// outputs, which may still lie in the 256 MB memory-side cache from what wrote
+// or read them, non-temporal ones past it (three sets in turn, ordinary against
+// non-temporal: 2 shards to 1 of 17 MB 8.4 against 10.7 us, 3 to 2 of 11 MB 10.1
+// against 12.0; 4 to 1 of 50 MB 45.7 against 42.6, 16 to 2 of 13 MB 43.5
+// against 40.8).
+constexpr uint64_t kRs8CachedBytes = 128u << 20;
+
 static int launch_mix(uint8_t* const* in, int nin, uint8_t* const* out, int nout,
                       const uint8_t* M /* nout x nin */, int64_t S, hipStream_t st,
                       const char* what) {
@@ -299,8 +313,11 @@ static int launch_mix(uint8_t* const* in, int nin, uint8_t* const* out, int nout
         const uint32_t nvec = uint32_t(S / 16);
         hipLaunchKernelGGL(kern.fn, dim3(blocks_for(nvec, kRs8BS * kern.vec)), dim3(kRs8BS), 0, st, pi, po, mix,
                            uint32_t(S), nvec);
-    } else if (fits_buffer(uint64_t(S))) {   // 32-bit columns
-        return launch_loop<kShards>(Rs8Io<kShards>{pi, po}, mix, nin, nout, uint32_t(S), st, what);
+    } else if (fits_buffer(uint64_t(S)) && nin * nout > 1) {   // 32-bit columns
+        const Rs8Io<kShards> io = {pi, po};
+        return uint64_t(nin + nout) * uint64_t(S) <= kRs8CachedBytes
+                       ? launch_loop<kShards, false>(io, mix, nin, nout, uint32_t(S), st, what)
+                       : launch_loop<kShards, true>(io, mix, nin, nout, uint32_t(S), st, what);
     } else {
         const uint64_t nvec = uint64_t(S) / 16;
         hipLaunchKernelGGL(gf8_mix_generic_kernel, dim3(unsigned((nvec + kRs8BS - 1) / kRs8BS)),
