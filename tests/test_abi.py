@@ -324,6 +324,83 @@ def test_written_buffers_must_not_alias(pkg, fake_ptrs):
     assert "pool overlaps P" in err()
 
 
+def test_kv_entries_refuse_on_the_host(pkg, fake_ptrs):
+    """The one-pass K/V entry points: a layout or stripe outside their limits is
+    KVEC_EUNSUPPORTED (the wrappers then take the copies), a wrong argument or
+    an overlap KVEC_EINVAL, all before any launch.  Fake addresses, 4 GiB apart;
+    every call below is refused."""
+    lib = pkg._lib
+    L = lib.lib()
+    G = 1 << 32
+    K, V, SH = G, 2 * G, 3 * G
+
+    def kv(k=K, v=V, B=1, H=8, T=512, D=256, sb=None, sh=None, st=None):
+        st = D if st is None else st
+        sh = T * D if sh is None else sh
+        sb = H * T * D if sb is None else sb
+        return lib.KvBhtd(k, v, B, H, T, D, sb, sh, st)
+
+    def backup(c, nd=8, S=None, shards=SH):
+        S = 2 * c.B * c.H * c.T * c.head_bytes // 2 // nd if S is None else S
+        return L.kvec_gs_rdp_backup_kv(c, shards, nd, S, 0, None)
+
+    def recover(c, nd=8, S=None, shards=SH, a=0, b=-1, star=0):
+        S = 2 * c.B * c.H * c.T * c.head_bytes // 2 // nd if S is None else S
+        return L.kvec_gs_rdp_recover_kv(shards, c, nd, S, star, a, b, None)
+
+    odd = [kv(k=K + 2), kv(v=V + 8), kv(D=40, st=40), kv(st=264), kv(sb=8, B=2), kv(st=-256), kv(T=0), kv(B=0), kv(D=8, st=8),
+           kv(T=1 << 20), kv(st=1 << 31), kv(T=1 << 40)]
+    for c in odd:
+        assert backup(c, S=1 << 20) == -2 and recover(c, S=1 << 20) == -2
+        assert L.kvec_kv_pack_bhtd(c, SH, 1 << 30, None) == -2
+        assert L.kvec_kv_unpack_bhtd(SH, 1 << 30, c, None) == -2
+    assert backup(kv(), nd=13) == -2 and recover(kv(), nd=17) == -2 and backup(kv(), nd=0, S=1 << 20) == -2
+    assert backup(kv(T=1, H=1), nd=8, S=63) == -2 and backup(kv(), S=-1) == -2
+    assert backup(kv(), S=(1 << 20) // 8 - 8) == -2               # the rows do not hold K and V
+    assert backup(kv(), shards=SH + 8) == -2 and recover(kv(), shards=SH + 8) == -2
+    assert backup(kv(), nd=12, S=1 << 27) == -2                   # row tensor past 2 GiB
+    assert L.kvec_kv_pack_bhtd(kv(), SH, (1 << 21) + 8, None) == -2
+    assert L.kvec_kv_pack_bhtd(kv(), SH, (1 << 21) - 16, None) == -2
+    assert L.kvec_kv_unpack_bhtd(SH, 1 << 31, kv(), None) == -2
+    assert backup(kv(k=None)) == -1 and backup(kv(), shards=None) == -1
+    assert backup(kv(k=SH + (1 << 20))) == -1 and b"overlaps k" in L.kvec_last_error()
+    assert recover(kv(v=SH)) == -1 and b"overlaps v" in L.kvec_last_error()
+    assert recover(kv(v=K + (1 << 20) - 16)) == -1 and b"k overlaps v" in L.kvec_last_error()
+    assert recover(kv(), a=0, b=3, star=-1) == -1 and b"star_base" in L.kvec_last_error()
+    assert L.kvec_kv_pack_bhtd(kv(), V, 1 << 21, None) == -1
+    assert L.kvec_kv_unpack_bhtd(SH, 1 << 21, kv(v=K), None) == -1 and b"k overlaps v" in L.kvec_last_error()
+
+    one = (C.c_int32 * 1)(0)
+    M = 1 << 20
+    for code in ("rs16", "rs8"):
+        size = (lambda b: b) if code == "rs8" else (lambda b: b // 2)
+
+        def enc(k=K, v=V, half=M, sh=SH, nk=8, m=2, row=M // 4):
+            return getattr(L, f"kvec_{code}_encode_kv")(k, v, half, sh, nk, m, size(row), None)
+
+        def rec(k=K, v=V, half=M, sh=SH, nk=8, m=2, row=M // 4, er=one, n=1):
+            return getattr(L, f"kvec_{code}_recover_kv")(sh, k, v, half, nk, m, size(row), er, n, None)
+
+        for kw in (dict(k=K + 8), dict(half=M - 8), dict(half=1 << 30, row=1 << 28), dict(sh=SH + 8), dict(half=0),
+                   dict(row=M // 4 - 16), dict(row=1 << 28)):
+            assert enc(**kw) == -2 and rec(**kw) == -2, (code, kw)
+        assert enc(m=5) == -2 and enc(m=0) == -2
+        assert rec(n=0) == -2
+        assert enc(k=None) == -1 and enc(sh=None) == -1 and rec(v=None) == -1 and rec(er=None) == -1
+        assert enc(k=SH + 3 * M // 2) == -1 and b"shards overlaps K" in L.kvec_last_error()
+        assert rec(v=K + M - 16) == -1 and b"K overlaps V" in L.kvec_last_error()
+        assert rec(er=(C.c_int32 * 1)(-1)) == -1 and rec(er=(C.c_int32 * 1)(10)) == -1
+        assert rec(m=1, er=(C.c_int32 * 2)(0, 1), n=2) == (-1 if code == "rs16" else -4)
+    # GF(2^16) rows: ascending data rows, up to 64 of them; rows under 64 words
+    assert L.kvec_rs16_recover_kv(SH, K, V, M, 8, 2, M // 8, (C.c_int32 * 2)(3, 3), 2, None) == -1
+    assert L.kvec_rs16_recover_kv(SH, K, V, M, 8, 2, M // 8, (C.c_int32 * 1)(8), 1, None) == -1
+    assert L.kvec_rs16_recover_kv(SH, K, V, M, 65, 2, M // 8, one, 1, None) == -2
+    assert L.kvec_rs16_encode_kv(K, V, 16, SH, 8, 2, 63, None) == -2
+    # GF(2^8) rows of whole 16 bytes, and the code's own limits
+    assert L.kvec_rs8_encode_kv(K, V, M, SH, 8, 2, M // 4 + 8, None) == -1
+    assert L.kvec_rs8_encode_kv(K, V, M, SH, 33, 1, M // 4, None) == -1
+
+
 def test_build_rejects_register_spills():
     """The build refuses kernels whose resource-usage remarks report spilled
     SGPRs or VGPRs; scratch without spills (a run-time indexed array) passes."""

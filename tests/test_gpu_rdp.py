@@ -245,6 +245,15 @@ def test_chain_decode_large_sets(pkg, ora, gpu, p, k, unit, past):
     _every_pattern(pkg, ora, gpu, p, k, (256 << 20) // ((k + 2) * (p - 1)) // 16 * 16 + past, unit)
 
 
+# shards of 2 to 4 GiB, the last of the chain decode's 32-bit offsets
+@pytest.mark.parametrize("p,k,R", [(3, 1, (1 << 31) - 16), (5, 2, (1 << 29) + 16), (7, 3, 715_827_872),
+                                   (11, 2, 429_496_720), (13, 1, 357_913_936)])
+@pytest.mark.parametrize("unit", [0, 65536])
+def test_chain_decode_up_to_4gib(pkg, ora, gpu, p, k, R, unit):
+    assert (1 << 31) < (p - 1) * R < (1 << 32)
+    _every_pattern(pkg, ora, gpu, p, k, R, unit)
+
+
 # shards of 4 GiB and more, which the codes without a compiled network decode by
 # the general map (p = 3 past the caches, above, does so for two of its patterns)
 @pytest.mark.parametrize("p,k,R", [(3, 1, (1 << 31) + 1040), (5, 2, (1 << 30) + 16), (7, 3, 715_827_904),
