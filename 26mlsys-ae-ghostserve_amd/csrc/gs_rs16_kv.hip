@@ -543,10 +543,13 @@ static void byte_maps(uint16_t c, uint32_t (&out)[kRs16Tab]) {
 }
 
 // One or two lost rows: 256 threads with four rows in flight, or 512 with two
-// from 8 MiB rows on (kernel trace, RS(6, 2), two rows lost: 5.5 MB rows 13.7
-// us either way, 0.7 MB 8.8 against 9.2; whole calls with 22 MB rows 57 against
-// 59-61 us).  More: bit planes, two rows of four windows in flight; 128 and 512
-// threads ran 39 and 43 against 35 us (16 rows of 4.2 MB, four lost).
+// from 8 MiB rows on.  Whole calls, 256 threads against 512: RS(4, 1) rows of 2 to
+// 7 MB 11.3-11.6 against 11.9-13.1 us, 9 MB 16.3 against 16.8, 22 MB 34.8 against
+// 33.9; RS(6, 2) 2 MB 12.6 against 13.1, 9 MB 25.6 against 26.6, 22 MB 56.9 against
+// 56.1; RS(10, 2) 30 MB 122.6 against 119.2.  They cross between 10 and 12 MB, so
+// rows of 8 to 11 MB give away up to 4 %.  More lost rows: bit planes, two rows of
+// four windows in flight; 128 and 512 threads ran 39 and 43 against 35 us (16 rows
+// of 4.2 MB, four lost).
 template <int M>
 static void rs_recover_launch(KvStream dst, uint8_t* sh, uint64_t sh_bytes, uint32_t Sb, int k, const int32_t* missing,
                               hipStream_t st) {
