@@ -174,7 +174,7 @@ __global__ __launch_bounds__(BS) void gs_recover_kv_kernel(uint8_t* sh, uint32_t
         acc ^= m ? funnel16(lo[i], from_next_lane_or(lo[i], e1[i]), m) : lo[i];
         const uint32_t r0 = A - t0;
         if (row_of(i) < ND && X >= r0 && X + 16 <= r0 + Sb && X + 16 <= out_len)
-            st_stream(kv_at<FLAT>(dst, X), 0, lo[i]);
+            kv_put<FLAT>(dst, X, lo[i]);
     }
     if (blockIdx.x == 0) {
         for (uint32_t u = threadIdx.x; u < 32 * ND; u += BS) {
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(kPackBS) void kv_rows_kernel(KvStream s, uint8_t* r
 #pragma unroll
         for (int n = 0; n < kPackN; ++n) {
             const uint32_t x = x0 + n * 1024 + lane16;
-            if (x < nbytes) st_stream(kv_at<FLAT>(s, x), 0, v[n]);
+            if (x < nbytes) kv_put<FLAT>(s, x, v[n]);
         }
     }
 }
