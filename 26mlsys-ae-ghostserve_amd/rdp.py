@@ -99,6 +99,15 @@ def _token_major(keys, values):
     return tuple(x.permute(2, 0, 1, 3).contiguous().view(x.shape[2], -1) for x in (keys, values))
 
 
+def _copies_are_faster(B: int, H: int, T: int, head_bytes: int) -> bool:
+    """Large K and V [B, H, T, head] of many heads of 16 bytes: each chunk that a
+    wave of the one-pass kernels moves is in another head's plane (backup of six
+    rows, K of 67 MB, copies against one pass: 128 heads 268 against 192 us, 256
+    heads 186 against 241, 1024 heads 172 against 217; 256 heads of 12 MB 63
+    against 55, 17 MB 75 against 77)."""
+    return head_bytes == 16 and B * H >= 192 and B * H * T * 16 >= 14_000_000
+
+
 def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
                          num_data_shards: int, star_base: int = 0, scheme: str = "ghostserve"):
     """benchmark/rdp/main.py:44-92: token-major pack + P/Q in one call.
@@ -124,10 +133,12 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
     else:
         shard_size, pad_words = determine_shard_size_words(total_words, nd)
     # one pass over K and V where they lie, when the layout allows it (what can
-    # be known here: up to twelve rows of 64 words and more); else token-major
-    # copies, then the pack and the code
+    # be known here: up to twelve rows of 64 words and more) and unless copies
+    # are faster (never when the tensors are token major already); else
+    # token-major copies, then the pack and the code
     kv = None
-    if scheme == "spec" or (nd <= 12 and shard_size >= 64):
+    if (scheme == "spec" or (nd <= 12 and shard_size >= 64)) and not (
+            _copies_are_faster(B, H, T, D * 2) and keys_bhtd.stride(2) != n):
         kv = _lib.kv_bhtd(keys_bhtd, values_bhtd)
     # (the copies first, so that the host prepares the rest behind them)
     copies = _token_major(keys_bhtd, values_bhtd) if kv is None else None
@@ -194,9 +205,11 @@ def fused_recovery_full_kv(pkg: dict, missing_a: int, missing_b: int = -1):
     _lib.require_cuda(shards, what="fused_recovery_full_kv tensor")
     # the rows written straight to K and V when the layout allows it (known
     # before they are allocated: heads of whole 16 bytes, rows of 64 words and
-    # more); else, and where n is not the shape's, through a token-major copy
+    # more) and unless copies are faster; else, and where n is not the shape's,
+    # through a token-major copy
     kv = None
-    if D * dtype.itemsize % 16 == 0 and (is_spec or shard_size >= 64) and n == B * H * D:
+    if (D * dtype.itemsize % 16 == 0 and (is_spec or shard_size >= 64) and n == B * H * D
+            and not _copies_are_faster(B, H, T, D * dtype.itemsize)):
         kv_shape = (int(B), int(H), int(T), int(D))
         keys = torch.empty(kv_shape, dtype=dtype, device=shards.device)
         values = torch.empty(kv_shape, dtype=dtype, device=shards.device)

@@ -202,6 +202,25 @@ def test_rs_wrappers_take_the_entry_points(pkg, gpu, monkeypatch, scheme, k, m, 
     assert all(torch.equal(x.view(torch.int16).cpu(), w) for x, w in zip((k2, v2), kv.want))
 
 
+# both sides of the lines past which many heads of 16 bytes are copied
+@pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
+@pytest.mark.parametrize("B,H,T,direct", [(1, 192, 4556, True), (1, 192, 4560, False), (1, 191, 4600, True), (5, 64, 3001, False)])
+def test_many_heads_of_16_bytes(pkg, ora, gpu, monkeypatch, scheme, B, H, T, direct):
+    kv = KV(pkg, gpu, "head", B, H, T, 8, T)
+    kv.fill()
+    took = []
+    real = pkg._lib.call_if_built
+    monkeypatch.setattr(pkg._lib, "call_if_built", lambda name, *a: took.append(real(name, *a)) or took[-1])
+    pk = pkg.rdp.fused_backup_full_kv(*(t.view(torch.float16) for t in kv.t), 5, scheme=scheme)
+    want = ora.gs_backup(*kv.tn(), 5, 0)
+    if scheme == "ghostserve":
+        assert np.array_equal(pk["shards_KV"].cpu().numpy(), want)
+    pk["shards_KV"].view(torch.int16)[3] = 0x5A5A
+    k2, v2, _ = pkg.rdp.fused_recovery_full_kv(pk, 3)
+    assert took == [True] * 2 * direct
+    assert all(torch.equal(x.view(torch.int16).cpu(), w) for x, w in zip((k2, v2), kv.want))
+
+
 # row tensors just below 2 GiB, K and V of 0.8 GB: 32-bit offsets near their end
 @pytest.mark.parametrize("H,D", [(1, 128), (8, 64)])
 def test_star_entries_near_2gib(pkg, gpu, H, D):
