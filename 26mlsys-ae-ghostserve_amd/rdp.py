@@ -134,11 +134,11 @@ def fused_backup_full_kv(keys_bhtd: torch.Tensor, values_bhtd: torch.Tensor,
         shard_size, pad_words = determine_shard_size_words(total_words, nd)
     # one pass over K and V where they lie, when the layout allows it (what can
     # be known here: up to twelve rows of 64 words and more) and unless copies
-    # are faster (never when the tensors are token major already); else
-    # token-major copies, then the pack and the code
+    # are faster (never when a token's heads are adjacent); else token-major
+    # copies, then the pack and the code
     kv = None
     if (scheme == "spec" or (nd <= 12 and shard_size >= 64)) and not (
-            _copies_are_faster(B, H, T, D * 2) and keys_bhtd.stride(2) != n):
+            _copies_are_faster(B, H, T, D * 2) and keys_bhtd.stride(1 if H > 1 else 0) != D):
         kv = _lib.kv_bhtd(keys_bhtd, values_bhtd)
     # (the copies first, so that the host prepares the rest behind them)
     copies = _token_major(keys_bhtd, values_bhtd) if kv is None else None

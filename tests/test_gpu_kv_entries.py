@@ -204,9 +204,12 @@ def test_rs_wrappers_take_the_entry_points(pkg, gpu, monkeypatch, scheme, k, m, 
 
 # both sides of the lines past which many heads of 16 bytes are copied
 @pytest.mark.parametrize("scheme", ["ghostserve", "spec"])
-@pytest.mark.parametrize("B,H,T,direct", [(1, 192, 4556, True), (1, 192, 4560, False), (1, 191, 4600, True), (5, 64, 3001, False)])
-def test_many_heads_of_16_bytes(pkg, ora, gpu, monkeypatch, scheme, B, H, T, direct):
-    kv = KV(pkg, gpu, "head", B, H, T, 8, T)
+@pytest.mark.parametrize("order,B,H,T,took_backup,took_recovery", [
+    ("head", 1, 192, 4556, True, True), ("head", 1, 192, 4560, None, None), ("head", 1, 191, 4600, True, True),
+    ("head", 5, 64, 3001, None, None), ("token", 5, 64, 3001, True, None), ("pool", 5, 64, 3001, True, None),
+    ("token", 200, 1, 4400, None, None), ("pool", 200, 1, 4400, True, None)])
+def test_many_heads_of_16_bytes(pkg, ora, gpu, monkeypatch, scheme, order, B, H, T, took_backup, took_recovery):
+    kv = KV(pkg, gpu, order, B, H, T, 8, T)
     kv.fill()
     took = []
     real = pkg._lib.call_if_built
@@ -217,7 +220,7 @@ def test_many_heads_of_16_bytes(pkg, ora, gpu, monkeypatch, scheme, B, H, T, dir
         assert np.array_equal(pk["shards_KV"].cpu().numpy(), want)
     pk["shards_KV"].view(torch.int16)[3] = 0x5A5A
     k2, v2, _ = pkg.rdp.fused_recovery_full_kv(pk, 3)
-    assert took == [True] * 2 * direct
+    assert took == [x for x in (took_backup, took_recovery) if x]
     assert all(torch.equal(x.view(torch.int16).cpu(), w) for x, w in zip((k2, v2), kv.want))
 
 
