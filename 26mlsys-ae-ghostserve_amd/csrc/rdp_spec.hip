@@ -135,9 +135,10 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // First the syndromes, as the encode folds its parities: row[r] is the XOR of
 // row r's surviving cells (P's included), diag[d] that of diagonal d's and of
 // Q[d].  Lost shards are read through an empty buffer resource (zeros, no
-// memory traffic), and so are the cells of diagonal p-1 when Q alone is lost,
-// which needs no row syndrome; nothing else here depends on the pattern and
-// every diagonal is a compile-time accumulator; the cells of rdp_group(p, k) shards are kept in
+// memory traffic), and so are, up to p = 7, the cells of diagonal p-1 when Q alone
+// is lost, which needs no row syndrome (one cell in p-1; past p = 7 the second
+// resource costs the other patterns 1 %); nothing else here depends on the
+// pattern and every diagonal is a compile-time accumulator; the cells of rdp_group(p, k) shards are kept in
 // flight, a shard's requested as an earlier one's are folded.  Then the lost cells, from the syndromes in LDS (each lane its
 // own column, no barrier), at offsets that follow from c0 and c1:
 //   two columns   the chains of the paper (FAST 2004, section 4): from the
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(kBS) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
                 return __builtin_amdgcn_make_buffer_rsrc(sh.p[s], (short)0, int(none ? 0u : nb), int(kBufWord3));
             };
             const bool none = (lost.absent >> s) & 1;
-            const __amdgpu_buffer_rsrc_t rs = view(none), ro = view(none || lost.c0 < 0);
+            const __amdgpu_buffer_rsrc_t rs = view(none), ro = view(none || (P <= 7 && lost.c0 < 0));
 #pragma unroll
             for (int r = 0; r < ROWS; ++r)
                 x[s % G][r] = __builtin_bit_cast(

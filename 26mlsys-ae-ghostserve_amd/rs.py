@@ -12,6 +12,7 @@ the reference.  Differences that change no output byte:
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 
 import numpy as np
@@ -240,11 +241,11 @@ def backwards_decode_kv(shards: torch.Tensor, meta: dict, missing_shards):
     # and the layout allows it
     if (one_pass and missing_data and rows_held >= num_data + len(missing_data) and
             avail_par[:len(missing_data)] == list(range(len(missing_data)))):
-        lost = np.asarray([int(i) for i in missing_data], dtype=np.int32)
+        lost = (ctypes.c_int32 * len(missing_data))(*missing_data)
         if _lib.call_if_built("kvec_rs16_recover_kv", shards.data_ptr(), K.data_ptr(), V.data_ptr(),
                               2 * int(N_k), int(num_data),
                               min(int(num_parity), rows_held - int(num_data)), int(shard_sz),
-                              lost.ctypes.data, len(missing_data), _stream(shards)):
+                              lost, len(missing_data), _stream(shards)):
             return K.view(B, H, T, D), V.view(B, H, T, D)
     if missing_data:
         if len(missing_data) > 16:
